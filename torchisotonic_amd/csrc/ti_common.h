@@ -171,9 +171,11 @@ __device__ __forceinline__ bool clip_passes(T v, bool use_lo, T lo, bool use_hi,
 // and 3) and row_bcast:31 (lane 31 into rows 2 and 3); lanes without a source keep the
 // identity (zero). Controls as in the GFX9 DPP encoding: row_shr:k 0x110 + k, wave_shr:1 0x138,
 // row_bcast:15 0x142, row_bcast:31 0x143.
+// (where every row is written, a lane without a source gets the zero from the instruction itself,
+// bound_ctrl, with no register cleared for it first)
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_i32(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, ROWS == 0xF);
 }
 
 template <int CTRL, int ROWS>
@@ -209,6 +211,20 @@ __device__ __forceinline__ double wave_incl_f64(double v) {
   v = dpp_f64<0x142, 0xA>(v) + v;
   v = dpp_f64<0x143, 0xC>(v) + v;
   return v;
+}
+
+// The largest of the lanes' values (none negative), in every lane.
+__device__ __forceinline__ double wave_max_f64(double v) {
+  v = __builtin_fmax(dpp_f64<0x111, 0xF>(v), v);
+  v = __builtin_fmax(dpp_f64<0x112, 0xF>(v), v);
+  v = __builtin_fmax(dpp_f64<0x114, 0xF>(v), v);
+  v = __builtin_fmax(dpp_f64<0x118, 0xF>(v), v);
+  v = __builtin_fmax(dpp_f64<0x142, 0xA>(v), v);
+  v = __builtin_fmax(dpp_f64<0x143, 0xC>(v), v);
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(b)), 63));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(b >> 32)), 63));
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 // The same in double-double, each step adding the lower lanes' part on the left.

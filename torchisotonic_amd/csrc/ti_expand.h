@@ -47,26 +47,34 @@ __device__ __forceinline__ int block_excl_i32(int v, int* wsum) {
   }
 }
 
-// The row's final hull h (row_bad: a NaN row) expanded by NT threads, with x.lds_bytes of LDS
-// at lds (at least expand_lds_min). The hull's vertices become a bitmap of the row's elements in
+// A final hull in the vertex store, for expand_hull: a vertex's index, an edge's differences.
+template <bool W>
+struct StoredHull {
+  VArr v;
+  __device__ __forceinline__ int idx(int k) const { return v.idx[k]; }
+  __device__ __forceinline__ void edge(int k, double& dW, double& dS) const {
+    vdiff<W>(vload<W>(v, k), vload<W>(v, k + 1), dW, dS);
+  }
+};
+
+// The row's final hull of cnt vertices, h (row_bad: a NaN row), expanded by nt threads (a
+// multiple of 64, at most NT), with
+// x.lds_bytes of LDS at lds (at least expand_lds_min, or room in the table for every edge). The hull's vertices become a bitmap of the row's elements in
 // LDS, and per bitmap word the vertices before it (one scan), from which an element's edge (the
 // vertices at or before it, less one) and a tile's records (its first and last edges, as
 // rank_kernel's searches find them) follow without a search; the start bits are the bitmap; the
-// fit, 16 * NT elements a pass, is each edge's slope rounded once, signed and clamped as the
+// fit, E * nt elements a pass, is each edge's slope rounded once, signed and clamped as the
 // expansion kernels form it, from a table of the edges' values in LDS, restaged where a pass needs
 // edges past the table (a row's hull can have a vertex every element). Each thread stores pieces
 // of 16 bytes, every store instruction of a wave on one contiguous 1 KiB.
-template <typename T, bool W, bool MAP, int NT>
-__device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, int64_t row, char* lds) {
-  constexpr int E = 16;              // elements a thread a pass
+template <typename T, bool W, bool MAP, int NT, int E, class H>
+__device__ void expand_hull(const RowExpand& x, const H& h, int cnt, bool row_bad, int64_t row, char* lds,
+                            int nt = NT) {
   constexpr int V = 16 / sizeof(T);  // elements a 16-byte store
   constexpr int G = E / V;           // stores a thread a pass
-  constexpr int kStep = E * NT;      // elements a pass
+  const int kStep = E * nt;          // elements a pass
   const int tid = threadIdx.x;
-  __syncthreads();  // the hull written (and repaired) by every thread, the LDS read
   const int n = static_cast<int>(x.n);
-  const int cnt = *h.count;
-  const VArr hv = dvarr_of(h);
   const int words = (n + 31) / 32;
   const int words4 = (words + 3) & ~3;
   int* wsum = reinterpret_cast<int*>(lds);  // (16 ints)
@@ -75,16 +83,16 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
   T* tab = reinterpret_cast<T*>(wpre + words4);
   const int cap = (x.lds_bytes - 64 - 2 * words4 * static_cast<int>(sizeof(uint32_t))) / static_cast<int>(sizeof(T));
   // the bitmap (a NaN row's too: its records come from its hull as any row's)
-  for (int k = tid; k < words; k += NT) vbits[k] = 0u;
+  for (int k = tid; k < words; k += nt) vbits[k] = 0u;
   __syncthreads();
-  for (int e = tid; e < cnt - 1; e += NT) {
-    const int p = hv.idx[e];
+  for (int e = tid; e < cnt - 1; e += nt) {
+    const int p = h.idx(e);
     atomicOr(&vbits[p >> 5], 1u << (p & 31));
   }
   __syncthreads();
   // vertices before each word: thread t counts words [t * wl, t * wl + wl)
   {
-    const int wl = (words + NT - 1) / NT;
+    const int wl = (words + nt - 1) / nt;
     const int k0 = min(tid * wl, words), k1 = min(k0 + wl, words);
     int c = 0;
     for (int k = k0; k < k1; ++k) c += __popc(vbits[k]);
@@ -99,10 +107,10 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
   auto below = [&](int i) { return wpre[i >> 5] + __popc(vbits[i >> 5] & ((1u << (i & 31)) - 1u)); };
   // the start bits (a NaN row: its first element only)
   if (x.starts != nullptr)
-    for (int k = tid; k < words; k += NT) x.starts[row * words + k] = row_bad ? (k == 0 ? 1u : 0u) : vbits[k];
+    for (int k = tid; k < words; k += nt) x.starts[row * words + k] = row_bad ? (k == 0 ? 1u : 0u) : vbits[k];
   // tile records: ra, the last vertex at or before the tile's first element; rb, the first at or
   // after its end (the row's end vertex, cnt - 1, for the last tile)
-  for (int64_t t = tid; t < x.tpr; t += NT) {
+  for (int64_t t = tid; t < x.tpr; t += nt) {
     const int ta = static_cast<int>(t * x.tile_n);
     const int tb = min(ta + x.tile_n, n);
     const bool at_vertex = (vbits[ta >> 5] >> (ta & 31)) & 1u;
@@ -116,7 +124,7 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
     r.unused = 0.0;
     if (!row_bad && r.rb == r.ra + 1) {
       double dW, dS;
-      vdiff<W>(vload<W>(hv, r.ra), vload<W>(hv, r.ra + 1), dW, dS);
+      h.edge(r.ra, dW, dS);
       r.slope = slope_div(dS, dW);
     }
     x.tiles[row * x.tpr + t] = r;
@@ -128,7 +136,7 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
   const int lim = static_cast<int>(xlen);
   if (row_bad) {
     const T nanv = quiet_nan<T>();
-    for (int i = tid; i < lim; i += NT) out[i] = nanv;
+    for (int i = tid; i < lim; i += nt) out[i] = nanv;
     return;
   }
   const T tsgn = static_cast<T>((x.flags & TI_INCREASING) ? 1.0 : -1.0);
@@ -137,9 +145,9 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
   const T lo = static_cast<T>(x.lo), hi = static_cast<T>(x.hi);
   auto stage = [&](int e0) {  // edges [e0, e0 + cap) of the row's cnt - 1
     const int e1 = min(cnt - 1, e0 + cap);
-    for (int e = e0 + tid; e < e1; e += NT) {
+    for (int e = e0 + tid; e < e1; e += nt) {
       double dW, dS;
-      vdiff<W>(vload<W>(hv, e), vload<W>(hv, e + 1), dW, dS);
+      h.edge(e, dW, dS);
       tab[e - e0] = clip(tsgn * static_cast<T>(slope_div(dS, dW)), use_lo, lo, use_hi, hi);
     }
   };
@@ -167,7 +175,7 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
     int cum[G];
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-      g0[j] = c + j * (NT * V) + tid * V;
+      g0[j] = c + j * (nt * V) + tid * V;
       const int ii = g0[j] < n ? g0[j] : c;
       wb[j] = vbits[ii >> 5] >> (ii & 31);
       cum[j] = wpre[ii >> 5] + __popc(vbits[ii >> 5] & ((1u << (ii & 31)) - 1u));
@@ -198,6 +206,14 @@ __device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, i
       }
     }
   }
+}
+
+// The same from the vertex store, E = 16 elements a thread a pass.
+template <typename T, bool W, bool MAP, int NT>
+__device__ void expand_row(const RowExpand& x, const NodeOut& h, bool row_bad, int64_t row, char* lds) {
+  __syncthreads();  // the hull written (and repaired) by every thread, the LDS read
+  const int cnt = *h.count;
+  expand_hull<T, W, MAP, NT, 16>(x, StoredHull<W>{dvarr_of(h)}, cnt, row_bad, row, lds);
 }
 
 }  // namespace

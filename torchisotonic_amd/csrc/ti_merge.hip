@@ -201,8 +201,6 @@ __global__ __launch_bounds__(NT) void merge_kernel(MergeArgs a, int cap_lds, int
   const int64_t c0 = j * kGroup;  // first child within the row
   const int nch = static_cast<int>(min<int64_t>(kGroup, a.in.npr - c0));
   const NodeOut pout = node_out(a.out, W, row * a.out.npr + j);
-  // (a first child's count of -1: the span kernel merged this group already)
-  if (*node_out(a.in, W, row * a.in.npr + c0).count < 0) return;
 
   // Children (first wave): counts, NaN flags, and offsets within the parent (double-double scan).
   if (tid < kWave) {
@@ -806,42 +804,30 @@ LongPlan long_plan(int64_t batch, int64_t n, bool weighted, bool lo) {
   p.lo = lo;
   const int64_t tn = tile_elems(weighted);
   p.tiles_per_row = (n + tn - 1) / tn;
-  // The longest span that still gives the span kernel about 2^17 lanes (two waves per SIMD),
-  // within [kSpanMin, kSpanMax]: long spans mean fewer hulls to merge, short ones more lanes.
+  // Spans, the units of the vertex store's slots: a group is kGroup of them, one workgroup of
+  // group_kernel. The longest that still give about 2^17 spans (2048 groups, enough workgroups to
+  // fill the GPU), within [kSpanMin, kSpanMax].
   int64_t span0 = kSpanMax;
   while (span0 > kSpanMin && batch * ((n + span0 - 1) / span0) < (int64_t{1} << 17)) span0 >>= 1;
-  // Where spans of up to kSpanMax make a row one group, and that still leaves 2^15 lanes, take
-  // them: the span kernel's group merge then finishes each row, and no merge launch follows
-  // (1000 rows of 5000 float64: 150 -> 108 us). The span is the row split 64 ways (rounded up
-  // to 4 elements, 16-byte aligned spans), so the wave's lanes are all busy and each span is as
-  // short as one group allows (1000 rows of 5000: spans of 80 on 63 lanes, not 128 on 40;
-  // float64 108 -> 93 us).
+  // Rows that spans of up to kSpanMax make one group (up to 16384 elements): one group a row, however
+  // few the rows: its workgroup finishes the row, where shorter groups take a merge launch and
+  // four more after it (20 rows of 5000: 43 us, in one launch and the check for overflows 21).
   int64_t one_group = (((n + kGroup - 1) / kGroup) + 3) & ~int64_t{3};
   if (one_group < kSpanMin) one_group = kSpanMin;
-  if (one_group <= kSpanMax && (n + one_group - 1) / one_group <= kGroup && batch * ((n + one_group - 1) / one_group) >= (int64_t{1} << 15))
-    span0 = span0 > one_group ? span0 : one_group;
-  // Rows of at most kSpanMax elements in batches of thousands: one span per row, so the span
-  // kernel runs one row per lane and 64 rows a wave (a wave per row would keep a few lanes busy;
-  // 100000 rows of 64: 0.93 ms that way), and the span hulls are the final hulls.
+  if (one_group <= kSpanMax) span0 = span0 > one_group ? span0 : one_group;
+  // Rows of at most kSpanMax elements in batches of thousands: one span per row, one row a lane
+  // (span_run), for rows of at most 64 elements or batches of 32768 rows or more, where the GPU
+  // has lanes enough without splitting rows (100000 rows of 64: 56 us, a wave a row 136; of 128:
+  // 103 and 149). Other rows of at most 2048 elements: a wave or a small workgroup a row; their
+  // spans (k of at least 8 elements, none empty) only lay out the store.
+  const bool packed = n <= kSpanMax && batch >= 8192 && (batch >= 32768 || n <= 64);
   if (n <= kSpanMax && batch >= 8192) {
     int64_t s = kSpanMin;
     while (s < n) s <<= 1;
     span0 = span0 > s ? span0 : s;
   }
-  // Rows of at most 2048 elements (which one wave's lanes cannot all share with spans of
-  // kSpanMin or more): several rows a wave, k lanes each (a power of two up to 32), the smallest
-  // k that gives about 2^17 lanes, each span at least 8 elements and none empty. Each row's k
-  // span hulls are merged in the wave (log2 k rounds), so the span kernel finishes the rows, with
-  // k times the lanes of one row per lane and no idle lanes (10000 rows of 256: 135 -> 89 us;
-  // 5000 rows of 100: 87 -> 49 us, float64 weighted 148 -> 44 us).
-  // Where that leaves spans longer than kSpanMin and the GPU short of lanes, one row a wave with
-  // spans of kSpanMin does better (shorter spans, the same idle SIMDs); and one row a lane
-  // ("packed", above) does better in batches of 32768 rows or more, or for rows of at most 64
-  // elements, where the GPU has lanes enough without splitting rows (100000 rows of 128: 117 us
-  // packed, 158 us two lanes a row; float64 weighted 200 and 314 us).
   p.rows_per_wave = 1;
-  const bool packed_better = n <= kSpanMax && batch >= 8192 && (batch >= 32768 || n <= 64);
-  if (n <= 2048 && !packed_better) {
+  if (n <= 2048 && !packed) {
     int64_t kmin = 1;
     while (kmin * kSpanMax < n) kmin <<= 1;
     int64_t k = kmin;
@@ -942,27 +928,26 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
   const bool W = t.w != nullptr;
   char* base = static_cast<char*>(ws);
   const NodeLevel fin = p.level(ws, p.levels);
-  // level 0: span hulls (and the first merge level, fused, where there is one)
-  // Float32 data: the final hulls made convex in their stored values. Rows of one merge level
-  // get theirs from the span kernel (or, for a multi-row wave's overflowing spans, the level-1
-  // launch), whose waves check and repair them in place (span_fold); a final level of two or
-  // more launches up has a merge workgroup for every row, which does it at its end (fold) where
-  // rows are enough to spread those workgroups over the GPU (one workgroup reading a hull of
-  // millions of vertices would take milliseconds); otherwise two launches after the merges do.
+  // Rows of one span: their hulls from span_run, one row a lane. Longer rows: level 1, the groups'
+  // hulls, from group_run, which also expands rows of one group (their tile records, start bits
+  // and fit), so nothing follows it.
+  // Float32 data: the final hulls convex in their stored values. A span's or a group's hull is
+  // built on those values; a final level of two or more has a merge workgroup for every row,
+  // which repairs its hull at its end (fold) where rows are enough to spread those workgroups
+  // over the GPU (one workgroup reading a hull of millions of vertices would take milliseconds);
+  // otherwise two launches after the merges do.
   const int repair_passes = (t.flags & TI_REPAIR_CHAIN) != 0 ? 0 : kRepairPasses;
-  const bool span_fold = !p.lo && p.levels == 1;
   const bool fold = !p.lo && p.levels >= 2 && batch_fills_gpu(t.batch);
-  // Rows of one merge level, one row a wave: the wave that builds a row's final hull also writes
-  // its tile records, start bits and fit (span_expand), so no rank or expansion launch follows.
-  const bool span_expand = p.levels == 1 && p.rows_per_wave == 1;
   TileRec* const recs_at = reinterpret_cast<TileRec*>(base + p.off_rank);
-  hipError_t e = span_run(t, p.level(ws, 0), p.span0, p.level(ws, p.levels >= 1 ? 1 : 0), p.rows_per_wave,
-                          span_fold ? 1 + repair_passes : 0, span_expand ? recs_at : nullptr);
+  const bool one_group = p.levels == 1;
+  hipError_t e = p.levels == 0 ? span_run(t, p.level(ws, 0))
+                               : group_run(t, p.level(ws, 0), p.span0, p.level(ws, 1),
+                                           one_group ? t.n : kGroup * p.span0, one_group ? recs_at : nullptr);
   if (e != hipSuccess) return e;
-  // the span kernel has read every weight (and set the flag if one is not positive)
+  // every weight has been read (and the flag set if one is not positive)
   if (t.weights_read != nullptr && (e = hipEventRecord(t.weights_read, t.stream)) != hipSuccess) return e;
   // (the weights' mark: stored by the first merge launch as it starts, or by a kernel of its own
-  // where no merge launch follows the span kernel)
+  // where no merge launch follows)
   uint32_t* pending_mark = t.weights_mark;
   // for a caller that keeps only the final hulls: a bound on their vertex counts, from the
   // counts of level keep_level once it is merged
@@ -984,15 +969,9 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     }
     return t.hulls_ready != nullptr ? hipEventRecord(t.hulls_ready, t.stream) : hipSuccess;
   };
-  if ((e = report(0)) != hipSuccess) return e;
-  bool expanded = false;  // (the final merge launch expanded the rows)
-  for (int l = 1; l <= p.levels; ++l) {
-    // (one row a wave: the span kernel merged every group, in LDS or, where its hulls do not
-    // fit, in the group's global array; a multi-row wave's overflowing spans wait for a launch)
-    if (l == 1 && p.rows_per_wave == 1) {
-      if ((e = report(l)) != hipSuccess) return e;
-      continue;
-    }
+  if ((e = report(0)) != hipSuccess || (e = report(1)) != hipSuccess) return e;
+  bool expanded = one_group;  // (or the final merge launch expanded the rows)
+  for (int l = 2; l <= p.levels; ++l) {
     MergeArgs m;
     m.in = p.level(ws, l - 1);
     m.out = p.level(ws, l);
@@ -1005,13 +984,11 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     // (64 noisy span hulls take 300-500) where there are thousands, else 256 or 1024 threads
     // and up to 56 KB of slots for the fewer, larger hulls of the upper levels.
     // (the final level of float32 data repairs its hulls in the merge launch: fold)
-    const int fix = (fold || span_fold) && l == p.levels ? 1 + repair_passes : 0;
+    const int fix = fold && l == p.levels ? 1 + repair_passes : 0;
     // The final level of rows enough to fill the GPU, one workgroup a row (dense rows whose
     // bitmap, counts and a pass's edges fit the launch's LDS): the workgroup expands its row.
-    // Only from the second level on: a first-level launch merges just the rows of multi-row
-    // waves whose spans overflowed, the span kernel's waves having finished the others.
     const bool last_fills =
-        l == p.levels && l >= 2 && batch_fills_gpu(t.batch) && grid >= 64 && t.map.rows == nullptr;
+        l == p.levels && batch_fills_gpu(t.batch) && grid >= 64 && t.map.rows == nullptr;
     RowExpand x{};
     x.n = t.n;
     x.out = t.out;
@@ -1080,9 +1057,8 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     if ((e = report(l)) != hipSuccess) return e;
   }
   if (pending_mark != nullptr && (e = mark_run(pending_mark, t.mark_value, t.stream)) != hipSuccess) return e;
-  if (!p.lo && p.levels >= 1 && !fold && !span_fold) {
-    // (float32 data: the final hulls convex in their stored values; span hulls, the final hulls
-    // of rows of one span, are exact and convex already). Enough check workgroups a row for a
+  if (!p.lo && p.levels >= 2 && !fold) {
+    // (float32 data: the final hulls convex in their stored values). Enough check workgroups a row for a
     // hull of every element (4096 vertices each), at most 256 a row, or about 4096 in all where
     // the rows are few (one row of 1e8 with 3.8e7 vertices: 290 us of checks at 256).
     static std::atomic<unsigned> calls{0};
@@ -1101,7 +1077,7 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (span_expand || expanded) return hipSuccess;
+  if (expanded) return hipSuccess;
   if (t.n <= kXpackMaxN) {
     // rows of one tile: records and fit together, whole rows a workgroup
     ExpandArgs x;

@@ -16,6 +16,7 @@
 // slot of L and last of R fix the bridge. The survivors then move down in one ordered compaction.
 #pragma once
 
+#include "ti_points.h"
 #include "ti_tile.h"
 
 namespace ti {
@@ -96,29 +97,6 @@ struct MergeRounds {
   int wflag[16];            // per wave: bit 0 some junction died, bit 1 some walk did not finish
   int wsum[4][16];
 };
-
-template <bool W, bool PR>
-__device__ __forceinline__ void hdiff(const HPt& a, const HPt& b, double& dS, double& dW) {
-  dS = b.s - a.s;
-  if constexpr (PR) dS += b.sl - a.sl;
-  if constexpr (W) {
-    dW = b.w - a.w;
-    if constexpr (PR) dW += b.wl - a.wl;
-  } else {
-    dW = static_cast<double>(b.i - a.i);
-  }
-}
-
-// c ? a : b, field by field (a select of whole structs would keep them in memory)
-__device__ __forceinline__ HPt hsel(bool c, const HPt& a, const HPt& b) {
-  HPt r;
-  r.i = c ? a.i : b.i;
-  r.s = c ? a.s : b.s;
-  r.sl = c ? a.sl : b.sl;
-  r.w = c ? a.w : b.w;
-  r.wl = c ? a.wl : b.wl;
-  return r;
-}
 
 template <bool W, bool PR>
 __device__ __forceinline__ bool hpools_nb(const HPt& a, const HPt& b, const HPt& c) {

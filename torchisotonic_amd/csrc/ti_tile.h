@@ -134,16 +134,17 @@ __host__ __device__ inline size_t vertex_store_bytes(int64_t slots, bool weighte
   return align256(c * 4) + align256(c * 8) * ((weighted ? 2 : 1) * (lo ? 2 : 1));
 }
 
-__host__ __device__ inline NodeOut node_out(const NodeLevel& L, bool weighted, int64_t k) {
+// Node j of row `row` (node row * npr + j of the level).
+__host__ __device__ inline NodeOut node_at(const NodeLevel& L, bool weighted, int64_t row, int64_t j) {
   NodeOut o;
   char* p = L.meta;
+  const int64_t k = row * L.npr + j;
   const size_t kk = static_cast<size_t>(L.K), c = static_cast<size_t>(L.slots);
   o.count = reinterpret_cast<int*>(p) + k;
   p += align256(kk * 4);
   o.bad = reinterpret_cast<int*>(p) + k;
   p += align256(kk * 4);
   o.tot = reinterpret_cast<double*>(p) + 4 * k;
-  const int64_t row = k / L.npr, j = k - row * L.npr;
   const int64_t v0 = (row * L.npr0 + j * L.spn) * L.r0;
   char* q = L.store;
   o.idx = reinterpret_cast<int*>(q) + v0;
@@ -161,6 +162,11 @@ __host__ __device__ inline NodeOut node_out(const NodeLevel& L, bool weighted, i
     if (L.lo) o.wlo = reinterpret_cast<double*>(q) + v0;
   }
   return o;
+}
+
+__host__ __device__ inline NodeOut node_out(const NodeLevel& L, bool weighted, int64_t k) {
+  const int64_t row = k / L.npr;
+  return node_at(L, weighted, row, k - row * L.npr);
 }
 
 // The stateless gradient (ti_grad): every element's block sums of g and w from the partition.
@@ -308,10 +314,20 @@ __device__ __forceinline__ bool hpools(const HPt& a, const HPt& b, const HPt& c)
   return pools<true>(dS1, dW1, dS2, dW2);
 }
 
-// Rows longer than 32 elements: one lane builds the hull of each span of span0 elements
-// (kSpanMin..kSpanMax, a multiple of 4, chosen per call so that the span kernel has enough
-// lanes), then
-// workgroups merge G neighbouring hulls at a time until one hull per row remains.
+// c ? a : b, field by field (a select of whole structs would keep them in memory)
+__device__ __forceinline__ HPt hsel(bool c, const HPt& a, const HPt& b) {
+  HPt r;
+  r.i = c ? a.i : b.i;
+  r.s = c ? a.s : b.s;
+  r.sl = c ? a.sl : b.sl;
+  r.w = c ? a.w : b.w;
+  r.wl = c ? a.wl : b.wl;
+  return r;
+}
+
+// Rows longer than 32 elements: spans of span0 elements (kSpanMin..kSpanMax, a multiple of 4,
+// chosen per call), groups of kGroup spans whose hulls one workgroup each builds, then workgroups
+// merge kGroup neighbouring hulls at a time until one hull per row remains.
 constexpr int kSpanMin = 32;
 constexpr int kSpanMax = 256;
 constexpr int kGroup = 64;
@@ -416,15 +432,15 @@ struct KeepPlan {
 KeepPlan keep_plan(int64_t batch, int64_t n, bool weighted, bool lo, int64_t maxc);
 hipError_t long_keep(const LongPlan& p, const void* ws, const KeepPlan& k, void* kept, hipStream_t stream);
 
-// Level 0 (span hulls) and, fused, level 1: a group whose hulls fit the wave's LDS is merged in
-// place into its level-1 node of `hulls1` and its first span's count set to -1. With
-// rows_per_wave > 1, each wave holds that many rows of spans_per_row spans (a power of two) and
-// merges each row's spans into the row's hull. fix > 0: those hulls are the rows' final hulls of
-// float32 data, made convex in their stored values by the same waves (fix - 1 removal passes).
-// tiles given (rows of one merge level, one row a wave): each wave also writes its row's fit,
-// start bits and tile records (into tiles), in place of the rank and expansion launches.
-hipError_t span_run(const TileArgs& t, const NodeLevel& hulls, int64_t span0, const NodeLevel& hulls1,
-                    int rows_per_wave, int fix, TileRec* tiles);
+// The final hulls of rows of one span (levels == 0), one row a lane: hulls is level 0.
+hipError_t span_run(const TileArgs& t, const NodeLevel& hulls);
+
+// Level 1 (or the rows' final hulls) from groups of g_elems elements, one workgroup a group:
+// out's nodes, one a group; spans: level 0, in whose slots a group of too many candidates builds
+// its chunks' hulls. tiles given (rows of one group): the workgroup also writes its row's fit,
+// start bits and tile records.
+hipError_t group_run(const TileArgs& t, const NodeLevel& spans, int64_t span0, const NodeLevel& out, int64_t g_elems,
+                     TileRec* tiles);
 
 // Backward of long rows, from the forward's final hulls and tile ranks (its workspace).
 struct LongGradArgs {
