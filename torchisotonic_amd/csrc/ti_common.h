@@ -260,6 +260,7 @@ __device__ __forceinline__ double wave_last_f64(double x) {
   const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(b >> 32)), 63));
   return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
+__device__ __forceinline__ int wave_last_i32(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
 __device__ __forceinline__ DD wave_last_dd(DD v) { return DD{wave_last_f64(v.hi), wave_last_f64(v.lo)}; }
 
 // floor(e / n) for e * n < 2^32 (e >= 0, n >= 1): the high word of e * ceil(2^32 / n), exact

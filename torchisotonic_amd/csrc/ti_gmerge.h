@@ -3,7 +3,6 @@
 #pragma once
 
 #include "ti_common.h"
-#include "ti_slots.h"
 #include "ti_tile.h"
 
 namespace ti {

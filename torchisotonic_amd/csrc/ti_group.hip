@@ -491,11 +491,6 @@ __global__ __launch_bounds__(NT, 4) void group_kernel(GroupArgs a) {
   uint64_t alive = nact == kWave ? ~uint64_t{0} : (uint64_t{1} << nact) - 1;
   auto wave_point = [&](int j) { return CPt{cs[c0 + j], cw[c0 + j]}; };
   if (nact > 0) alive = coarse_rounds(alive, me, wave_point);
-  auto at_or_below = [](uint64_t m, int j) { return 63 - __builtin_clzll(m & ((uint64_t{2} << j) - 1)); };
-  auto beyond = [](uint64_t m, int j) {
-    const uint64_t h = (m >> j) >> 1;
-    return h ? j + 1 + __builtin_ctzll(h) : kWave;
-  };
   CPt ca{0.0, 0.0}, cb{0.0, 1.0};  // the chord over the thread's elements
   bool own = true;                 // (the wave's own)
   if constexpr (NW > 1) {

@@ -2,16 +2,15 @@
 //
 // Replaces the reference's chunk-start prefix, merge rounds and fit stages (reference
 // src/torchisotonic/csrc/tiles.cuh:1680-1725, 1524-1537 + 1728-1743, 1541-1667): instead of
-// one launch per pairwise round over segment lists, a workgroup merges G = 64 neighbouring
-// hulls at a time, six rounds in LDS, so a row of 1e8 elements (390,625 span hulls of 256
-// elements) needs four merge launches.
+// one launch per pairwise round over segment lists, a workgroup merges 64 neighbouring
+// hulls at a time in LDS, so a row of 1e8 elements (6104 groups of 16384) needs three merge
+// launches.
 //
-//   merge_kernel   G child hulls (compact arrays, double-double coordinates relative to the
-//                  child) -> one parent hull relative to the parent. Children are laid end to
-//                  end with their shared boundary point stored once, so a merge whose junction
-//                  is already convex moves nothing; a bridge moves the right part's surviving
-//                  suffix down. Works in LDS when the children's vertices fit (the case for
-//                  noisy data, where hulls are small), else in the parent's own global array.
+//   merge_kernel   up to 64 child hulls (compact arrays, coordinates relative to the child) -> one
+//                  parent hull relative to the parent: nearly every vertex lies above a chord of
+//                  the children's first points and is dropped as it is read; rounds of exact
+//                  tests in LDS leave the hull. In the parent's own global array where more are
+//                  left than LDS holds (near-monotone data).
 //   expand_kernel  per tile of the row (four to a workgroup): the final hull's vertices around
 //                  the tile (ranks from rank_kernel), edge slopes in float64 rounded once, every
 //                  element the slope of its edge with the clamp fused, and the start bits. y is
@@ -23,8 +22,8 @@
 #include "ti_common.h"
 #include "ti_expand.h"
 #include "ti_kernels.h"
-#include "ti_slots.h"
 #include "ti_gmerge.h"
+#include "ti_points.h"
 #include "ti_tile.h"
 
 namespace ti {
@@ -128,58 +127,131 @@ __global__ __launch_bounds__(kRepairThreads) void repair_kernel(NodeLevel fin, u
   if (tid == 0) *o.count = cnt;
 }
 
-// Per merge: the children (vertex counts, first slots, offsets within the parent) and the
-// fallback's pairwise-round bookkeeping.
-// The merge in LDS: the children's vertices into slots (every thread's loads in flight
-// together), the pairwise rounds, and the survivors out to the parent's arrays.
-template <bool W, bool PR, int NT, int G>
-__device__ void merge_lds(const MergeArgs& a, const MergeSmall& sm, MergeRounds& rs, const Slots<W, PR>& v,
-                          int64_t row, int64_t c0, int nch, const NodeOut& pout) {
-  const int tid = threadIdx.x;
+// Fewer slots go to the exact tests without chords (4000 rows of 16384 to 65536 elements, four
+// children of about 30 vertices each: the chords took 4 us of a 74 us launch).
+constexpr int kChordSlots = 256;
+
+// The chord under each child's vertices (a point and the slope), from a rough hull of the
+// children's first points, and the counts of the vertices it leaves, for merge_lds.
+struct MergeChords {
+  double cs[kGroup + 1], cw[kGroup + 1];  // the children's first points, and the parent's end
+  double s[kGroup], w[kGroup], m[kGroup], scale[kGroup];
+  int count[2][8][16];
+  int wc[16];
+  int result;
+};
+
+// By the first wave, once the children's totals are scanned (es, ew: the offsets of lane c's child).
+template <bool W>
+__device__ __forceinline__ void merge_chords(MergeChords& mc, int nch, DD es, DD ew, DD end_s, DD end_w) {
+  const int lane = threadIdx.x;
+  const CPt me{es.hi, ew.hi};
+  mc.cs[lane] = me.s;
+  mc.cw[lane] = me.w;
+  if (lane == 0) {
+    mc.cs[kGroup] = end_s.hi;
+    mc.cw[kGroup] = end_w.hi;
+  }
+  wave_fence();
+  auto point = [&](int c) { return CPt{mc.cs[c], mc.cw[c]}; };
+  const uint64_t alive =
+      coarse_rounds(nch == kGroup ? ~uint64_t{0} : (uint64_t{1} << nch) - 1, me, point);
+  if (lane < nch) {
+    const CPt a = point(at_or_below(alive, lane)), b = point(beyond(alive, lane));
+    const double m = slope_div(b.s - a.s, b.w - a.w);
+    mc.s[lane] = a.s;
+    mc.w[lane] = a.w;
+    mc.m[lane] = m;
+    // (what a height over the chord is made of, but for the vertex's own sum)
+    mc.scale[lane] = __builtin_fabs(a.s) + __builtin_fabs(b.s) + __builtin_fabs(m) * end_w.hi;
+  }
+}
+
+// The merge in LDS. The children's vertices laid end to end, their shared boundary points stored
+// once (slot s of child c: vertex s - off[c]); every vertex clearly above its child's chord is
+// dropped as it is read, the others compacted into the cap point slots, in order; rounds of exact
+// tests (prune) leave the parent's hull. False where more than cap are left by the chords (nothing
+// written then). A vertex's height over the chord is formed from its sums in the parent's frame
+// rounded to float64, with a margin of 2^-44 of all that goes into it.
+//
+// What bounds it: latency, three round trips to memory and about five rounds of tests, 4-12 us a
+// level; merging neighbouring hulls pairwise in six rounds of walks took 37-45 us (one row of 1e8:
+// 36 + 45 + 11 us for its three levels).
+template <bool W, bool PR, int NT>
+__device__ bool merge_lds(const MergeArgs& a, const MergeSmall& sm, MergeChords& mc, const Points<W, PR, int>& v,
+                          int cap, int64_t row, int64_t c0, int nch, const NodeOut& pout) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = wave_index();
+  constexpr int NW = NT / kWave;
   const int total = sm.total;
+  const bool chords = total > kChordSlots;
   // slots per thread with their loads in flight together (fewer in large workgroups, whose
   // threads have fewer registers and fewer slots each)
   constexpr int B = NT >= 1024 ? 2 : NT >= 256 ? 4 : 8;
+  int out = 0, buf = 0;
   for (int s0 = 0; s0 < total; s0 += NT * B) {
     HPt p[B];
-    int cs[B];
+    bool keep[B];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
       // (slots past the end load the last slot again, so the loads need no branches)
       const int s = min(s0 + u * NT + tid, total - 1);
-      cs[u] = child_of_slot(sm, nch, s);
-      p[u] = child_vertex<W, PR>(a, sm, row, c0, cs[u], s - sm.off[cs[u]]);
-    }
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int s = s0 + u * NT + tid;
-      if (s < total) {
-        sput(v, s, p[u]);
-        v.cid[s] = static_cast<uint8_t>(cs[u]);
+      const int c = child_of_slot(sm, nch, s);
+      p[u] = child_vertex<W, PR>(a, sm, row, c0, c, s - sm.off[c]);
+      keep[u] = s0 + u * NT + tid < total;
+      if (chords && s != 0 && s != total - 1) {
+        const double x = W ? p[u].w : static_cast<double>(p[u].i);
+        const double d = (p[u].s - mc.s[c]) - mc.m[c] * (x - mc.w[c]);
+        keep[u] = keep[u] && !(d > (__builtin_fabs(p[u].s) + mc.scale[c]) * 0x1p-44);
       }
     }
+    int at[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const uint64_t m = __ballot(keep[u]);
+      at[u] = __popcll(m & ((uint64_t{1} << lane) - 1));
+      if (lane == 0) mc.count[buf][u][wave] = __popcll(m);
+    }
+    if constexpr (NT == kWave) wave_fence();
+    else __syncthreads();
+    // (the other buffer next: a wave writes it only after every wave has read this one's
+    // predecessor)
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      int before = out;
+      for (int q = 0; q < NW; ++q) {
+        const int n = mc.count[buf][u][q];
+        before += q < wave ? n : 0;
+        out += n;
+      }
+      if (keep[u] && before + at[u] < cap) pput(v, before + at[u], p[u]);
+    }
+    buf ^= 1;
   }
-  for (int c = tid; c < nch; c += NT) rs.seg[0][c] = sm.off[c] + sm.cnt[c] - 1;
+  if (out > cap) {
+    __syncthreads();
+    return false;
+  }
   __syncthreads();
-  const int count = merge_rounds<W, PR, NT, G>(v, rs, total, nch);
+  const int count = prune_all<NT>(v, out, mc.wc, &mc.result);
   for (int s = tid; s < count; s += NT) {
-    const HPt x = sget(v, s);
+    const HPt x = pget(v, s);
     pout.idx[s] = x.i;
     put_dd(pout.shi, pout.slo, s, x.s, x.sl);
     if constexpr (W) put_dd(pout.whi, pout.wlo, s, x.w, x.wl);
   }
   if (tid == 0) *pout.count = count;
+  return true;
 }
 
-// One workgroup of NT threads per parent node: G = 64 children (fewer at a row's end) -> the
-// parent's hull. NT grows where few parents share the GPU (the upper levels), so that their
-// larger hulls still take few slots per thread.
 // Rows enough for their final merge workgroups to read their hulls at the GPU's bandwidth.
 constexpr bool batch_fills_gpu(int64_t batch) { return batch >= 256; }
 
 // LDS repair_row takes with NT threads (carved from a merge kernel's slots once they are free).
 constexpr size_t repair_lds_bytes(int nt) { return (nt + 2) * sizeof(VPt) + (nt / kWave + 1) * sizeof(int); }
 
+// One workgroup of NT threads per parent node: kGroup children (fewer at a row's end) -> the
+// parent's hull. NT grows where few parents share the GPU (the upper levels), so that their
+// larger hulls still take few slots per thread.
 // fix > 0: the launch makes the final hulls of float32 data, which the workgroup then makes convex
 // in their stored values (repair_row, with fix - 1 removal passes before its chain), so no check
 // launch follows.
@@ -187,10 +259,10 @@ constexpr size_t repair_lds_bytes(int nt) { return (nt + 2) * sizeof(VPt) + (nt 
 // workgroup then expands its row's final hull too (expand_row, with x.lds_bytes of its dynamic
 // LDS), in place of the rank and expansion launches.
 // DF: a deferring level, tab its parents' DeferTabs (see merge_global).
-template <bool W, bool PR, int NT, int G, typename TX = void, bool DF = false>
+template <bool W, bool PR, int NT, typename TX = void, bool DF = false>
 __global__ __launch_bounds__(NT) void merge_kernel(MergeArgs a, int cap_lds, int fix, RowExpand x, DeferTab* tab) {
   __shared__ MergeSmall sm;
-  __shared__ MergeRounds rs;
+  __shared__ MergeChords mc;
   extern __shared__ __align__(16) char lds_dyn[];
   const int tid = threadIdx.x;
   if (DF && tid == 0) tab[blockIdx.x].deferred = 0;
@@ -235,12 +307,14 @@ __global__ __launch_bounds__(NT) void merge_kernel(MergeArgs a, int cap_lds, int
       sm.total = islot + 1;  // slots
     }
     if (lane == 0) sm.bad = anybad;
+    if (wave_last_i32(islot) >= kChordSlots) merge_chords<W>(mc, nch, es, ew, wave_last_dd(is), wave_last_dd(iw));
   }
   __syncthreads();
 
-  if (sm.total <= cap_lds) {
-    merge_lds<W, PR, NT, G>(a, sm, rs, slots_carve<W, PR>(lds_dyn, cap_lds), row, c0, nch, pout);
-  } else {
+  // (children of more than four times the slots' vertices are hulls that keep most points: their
+  // chords drop few)
+  if (sm.total > 4 * cap_lds ||
+      !merge_lds<W, PR, NT>(a, sm, mc, points_carve<W, PR, int>(lds_dyn, cap_lds), cap_lds, row, c0, nch, pout)) {
     __shared__ MergeRanges mr;
     merge_global<W, PR, NT, DF>(a, sm, mr.rlo, mr.rhi, mr.pre, row, c0, nch, pout, DF ? tab + blockIdx.x : nullptr);
   }
@@ -981,7 +1055,7 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     pending_mark = nullptr;
     const unsigned grid = static_cast<unsigned>(t.batch * p.npr[l]);
     // Workgroup size and LDS slots by how many merges share the GPU: one wave and 768 slots
-    // (64 noisy span hulls take 300-500) where there are thousands, else 256 or 1024 threads
+    // where there are thousands, else 256 or 1024 threads
     // and up to 56 KB of slots for the fewer, larger hulls of the upper levels.
     // (the final level of float32 data repairs its hulls in the merge launch: fold)
     const int fix = fold && l == p.levels ? 1 + repair_passes : 0;
@@ -1035,10 +1109,10 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
       }
     };
 #define TI_MERGE_LAUNCH(Wv, PRv)                                                                            \
-  launch(merge_kernel<Wv, PRv, 64, 4>, merge_kernel<Wv, PRv, 256, 2>, merge_kernel<Wv, PRv, 1024, 2>,           \
-         merge_kernel<Wv, PRv, 64, 4, float>, merge_kernel<Wv, PRv, 256, 2, float>,                            \
-         merge_kernel<Wv, PRv, 64, 4, double>, merge_kernel<Wv, PRv, 256, 2, double>,                           \
-         merge_kernel<Wv, PRv, 256, 2, void, true>, merge_kernel<Wv, PRv, 1024, 2, void, true>, slot_bytes<Wv, PRv>())
+  launch(merge_kernel<Wv, PRv, 64>, merge_kernel<Wv, PRv, 256>, merge_kernel<Wv, PRv, 1024>,           \
+         merge_kernel<Wv, PRv, 64, float>, merge_kernel<Wv, PRv, 256, float>,                            \
+         merge_kernel<Wv, PRv, 64, double>, merge_kernel<Wv, PRv, 256, double>,                           \
+         merge_kernel<Wv, PRv, 256, void, true>, merge_kernel<Wv, PRv, 1024, void, true>, point_bytes<Wv, PRv, int>())
     // (node arrays and slots are double-double for both dtypes: see child_vertex)
     if (W) TI_MERGE_LAUNCH(true, true);
     else TI_MERGE_LAUNCH(false, true);

@@ -210,6 +210,15 @@ __device__ __forceinline__ uint64_t coarse_rounds(uint64_t alive, CPt me, G get)
   return alive;
 }
 
+// The last point of the mask at or below j; the first beyond j (the end point, 64, where none is).
+__device__ __forceinline__ int at_or_below(uint64_t m, int j) {
+  return 63 - __builtin_clzll(m & ((uint64_t{2} << j) - 1));
+}
+__device__ __forceinline__ int beyond(uint64_t m, int j) {
+  const uint64_t h = (m >> j) >> 1;
+  return h ? j + 1 + __builtin_ctzll(h) : kWave;
+}
+
 // The hull of points [0, cnt): its count, in every thread.
 template <int NT, bool W, bool PR, typename I>
 __device__ __forceinline__ int prune_all(const Points<W, PR, I>& pts, int cnt, int* wc, int* result, int nt = NT) {
