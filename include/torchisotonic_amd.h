@@ -410,6 +410,25 @@ int ti_interp_index(const void* xp, int64_t m, int dtype, void* index, size_t in
 int ti_interp_indexed(const void* x, const void* xp, const void* fp, const void* index,
                       size_t index_bytes, void* out, int64_t n, int64_t m, int dtype, void* stream);
 
+/* The calibration step before a fit: each run of equal keys (n of them, sorted; a NaN key equals
+ * none) pooled into one point, its key, its values' (weighted) mean and its total weight (its
+ * count without weights), as scikit-learn pools duplicate X (reference examples/ctr_calibration/
+ * calibrate.py:171-187). Sums in float64, in a fixed order.
+ *
+ * ti_pool_bytes: the workspace for n keys (n < 2^40; 256-byte aligned).
+ * ti_pool_count: the runs of `keys` (key_dtype), and whether each of the n weights `w` (dtype; or
+ *   NULL) is positive; the workspace then begins with two int64, the runs and 1 if a weight is not
+ *   positive (else 0), once the stream's work is done.
+ * ti_pool: with the same keys and workspace after it, the points. order[i] is the element (of y
+ *   and w, both of dtype) that has sorted key i; xp, mean, weight: knots (the runs counted)
+ *   float64 each; inverse: per sorted key its run, or NULL. */
+int ti_pool_bytes(int64_t n, size_t* bytes);
+int ti_pool_count(const void* keys, const void* w, int64_t n, int key_dtype, int dtype,
+                  void* workspace, size_t workspace_bytes, void* stream);
+int ti_pool(const void* keys, const int64_t* order, const void* y, const void* w, int64_t n,
+            int key_dtype, int dtype, void* workspace, size_t workspace_bytes, int64_t knots,
+            double* xp, double* mean, double* weight, int64_t* inverse, void* stream);
+
 /* Test hook: the starts bit array of a [batch, n] set as bytes (0/1), row-major - the
  * reference's bool starts tensor (reference tests/test_cuda.py:176 reads it). */
 int ti_starts_to_bool(const uint32_t* starts, uint8_t* out, int64_t batch, int64_t n,

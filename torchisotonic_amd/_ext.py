@@ -66,6 +66,9 @@ SYMBOLS = (
     "ti_interp_index_bytes",
     "ti_interp_index",
     "ti_interp_indexed",
+    "ti_pool_bytes",
+    "ti_pool_count",
+    "ti_pool",
     "ti_starts_to_bool",
 )
 
@@ -142,6 +145,12 @@ def load() -> ctypes.CDLL:
     lib.ti_interp_index.argtypes = [_vp, _i64, _int, _vp, _sz, _vp]
     lib.ti_interp_indexed.restype = _int
     lib.ti_interp_indexed.argtypes = [_vp] * 4 + [_sz, _vp, _i64, _i64, _int, _vp]
+    lib.ti_pool_bytes.restype = _int
+    lib.ti_pool_bytes.argtypes = [_i64, ctypes.POINTER(_sz)]
+    lib.ti_pool_count.restype = _int
+    lib.ti_pool_count.argtypes = [_vp, _vp, _i64, _int, _int, _vp, _sz, _vp]
+    lib.ti_pool.restype = _int
+    lib.ti_pool.argtypes = [_vp] * 4 + [_i64, _int, _int, _vp, _sz, _i64] + [_vp] * 5
     lib.ti_starts_to_bool.restype = _int
     lib.ti_starts_to_bool.argtypes = [_vp, _vp, _i64, _i64, _vp]
     got = lib.ti_abi_version()
@@ -419,6 +428,34 @@ def interp(x: Tensor, xp: Tensor, fp: Tensor, index: Tensor | None = None) -> Te
                                       xc.numel(), xpc.numel(), dtype, _stream(xc))
     _check(rc, "interp")
     return out
+
+
+def pool_sorted(
+    keys: Tensor, order: Tensor, y: Tensor, w: Tensor | None, want_inverse: bool
+) -> tuple[Tensor, Tensor, Tensor, Tensor | None]:
+    """Runs of equal sorted ``keys`` pooled (ti_pool): each run's key, the (weighted) mean of its
+    values and its total weight, float64, and each sorted key's run if ``want_inverse``.
+    ``order`` (int64) gives each sorted key's element of ``y`` and ``w`` (1-D, of one dtype, at
+    least as long as ``keys``). A ValueError where a weight is not positive."""
+    _on_gpu(keys, "keys")
+    kd, dtype = _dtype_code(keys), _dtype_code(y)
+    keys, order, y = keys.contiguous(), order.contiguous(), y.contiguous()
+    w = None if w is None else w.contiguous()
+    n, lib, nbytes = keys.numel(), load(), _sz()
+    _check(lib.ti_pool_bytes(n, ctypes.byref(nbytes)), "pool")
+    work = torch.empty(nbytes.value, dtype=torch.uint8, device=keys.device)
+    with _on_device(keys.device):
+        rc = lib.ti_pool_count(_ptr(keys), _ptr(w), n, kd, dtype, _ptr(work), work.numel(), _stream(keys))
+        _check(rc, "pool")
+        knots, bad = work[:16].view(torch.int64).tolist()
+        if bad:
+            raise ValueError("weight must be strictly positive")
+        xp, mean, weight = (torch.empty(knots, dtype=torch.float64, device=keys.device) for _ in range(3))
+        inverse = torch.empty(n, dtype=torch.int64, device=keys.device) if want_inverse else None
+        rc = lib.ti_pool(_ptr(keys), _ptr(order), _ptr(y), _ptr(w), n, kd, dtype, _ptr(work), work.numel(), knots,
+                         _ptr(xp), _ptr(mean), _ptr(weight), _ptr(inverse), _stream(keys))
+    _check(rc, "pool")
+    return xp, mean, weight, inverse
 
 
 def starts_to_bool(starts: Tensor, batch: int, n: int) -> Tensor:

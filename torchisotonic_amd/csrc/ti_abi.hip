@@ -596,6 +596,45 @@ int ti_interp_indexed(const void* x, const void* xp, const void* fp, const void*
                   "interp");
 }
 
+int ti_pool_bytes(int64_t n, size_t* bytes) {
+  if (bytes == nullptr) return fail(TI_EINVAL, "null pointer");
+  if (n < 1) return fail(TI_EINVAL, "need n >= 1 keys, got %lld", (long long)n);
+  if (n >= (int64_t{1} << 40)) return fail(TI_ESIZE, "%lld keys exceed the limit of 2^40 - 1", (long long)n);
+  *bytes = ti::pool_bytes(n);
+  return ok();
+}
+
+namespace {
+int check_pool(const void* keys, const void* work, size_t work_bytes, int64_t n, int key_dtype, int dtype) {
+  for (const int d : {key_dtype, dtype})
+    if (d != TI_F32 && d != TI_F64) return fail(TI_EDTYPE, "dtype must be TI_F32 or TI_F64, got %d", d);
+  size_t need = 0;
+  if (int rc = ti_pool_bytes(n, &need)) return rc;
+  if (keys == nullptr || work == nullptr) return fail(TI_EINVAL, "null pointer");
+  if (work_bytes < need) return fail(TI_EWORKSPACE, "workspace of %zu bytes, need %zu", work_bytes, need);
+  if ((reinterpret_cast<uintptr_t>(work) & 255) != 0) return fail(TI_EINVAL, "workspace must be 256-byte aligned");
+  return TI_OK;
+}
+}  // namespace
+
+int ti_pool_count(const void* keys, const void* w, int64_t n, int key_dtype, int dtype, void* workspace,
+                  size_t workspace_bytes, void* stream) {
+  if (int rc = check_pool(keys, workspace, workspace_bytes, n, key_dtype, dtype)) return rc;
+  return launched(ti::pool_count(keys, w, n, key_dtype, dtype, workspace, static_cast<hipStream_t>(stream)), "pool");
+}
+
+int ti_pool(const void* keys, const int64_t* order, const void* y, const void* w, int64_t n, int key_dtype, int dtype,
+            void* workspace, size_t workspace_bytes, int64_t knots, double* xp, double* mean, double* weight,
+            int64_t* inverse, void* stream) {
+  if (int rc = check_pool(keys, workspace, workspace_bytes, n, key_dtype, dtype)) return rc;
+  if (order == nullptr || y == nullptr || xp == nullptr || mean == nullptr || weight == nullptr)
+    return fail(TI_EINVAL, "null pointer");
+  if (knots < 1 || knots > n) return fail(TI_EINVAL, "need 1 <= knots <= n, got %lld", (long long)knots);
+  return launched(ti::pool(keys, order, y, w, n, key_dtype, dtype, workspace, knots, xp, mean, weight, inverse,
+                           static_cast<hipStream_t>(stream)),
+                  "pool");
+}
+
 int ti_starts_to_bool(const uint32_t* starts, uint8_t* out, int64_t batch, int64_t n, void* stream) {
   if (batch < 0 || n < 0) return fail(TI_EINVAL, "negative size");
   if (batch == 0 || n == 0) return ok();

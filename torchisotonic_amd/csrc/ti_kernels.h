@@ -52,6 +52,14 @@ size_t interp_index_bytes(int64_t m);
 hipError_t interp_index(const void* xp, int64_t m, int dtype, void* index, hipStream_t stream);
 hipError_t interp_indexed(const void* x, const void* xp, const void* fp, const void* index, size_t index_bytes,
                           void* out, int64_t n, int64_t m, int dtype, hipStream_t stream);
+// Runs of equal sorted keys pooled: the scratch for n keys; the runs counted (and w checked); each
+// run's key, mean and total weight written (see ti_pool).
+size_t pool_bytes(int64_t n);
+hipError_t pool_count(const void* keys, const void* w, int64_t n, int key_dtype, int dtype, void* work,
+                      hipStream_t stream);
+hipError_t pool(const void* keys, const int64_t* order, const void* y, const void* w, int64_t n, int key_dtype,
+                int dtype, void* work, int64_t knots, double* xp, double* mean, double* weight, int64_t* inverse,
+                hipStream_t stream);
 
 // Ragged rows of at most max_len (<= kShortMax) elements: row r is y[offsets[r], offsets[r + 1]).
 struct RaggedArgs {
