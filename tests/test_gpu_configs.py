@@ -27,8 +27,8 @@ def grads(y, w, c, **kw):
 
 
 def test_c1_plumbing() -> None:
-    # [1000, 5000] float32, 0.001 i + N(0, 1), unweighted, increasing: one wave per row, its
-    # lanes' spans merged in the span kernel
+    # [1000, 5000] float32, 0.001 i + N(0, 1), unweighted, increasing: one workgroup per
+    # row, the row one group
     print("config c1", flush=True)
     rng = np.random.default_rng(0)
     y = (0.001 * np.arange(5000) + rng.standard_normal((1000, 5000))).astype(np.float32)

@@ -190,9 +190,8 @@ def test_float32_store_rounding_keeps_the_fit_monotone() -> None:
 
 
 # (batch, n, merge levels): rows through two merge levels, fewer or more than 256 of them, and
-# rows whose final hulls the span kernel makes, one row a wave (merged by reference to the span
-# hulls, which do not fit the wave's LDS) or two rows a wave (the overflowing waves' rows merged
-# by the first merge launch)
+# rows of one group, whose candidates overflow the workgroup's LDS (chunks merged by reference) or
+# fit it
 STORE_ROUNDING_SHAPES = [(80, 100_000, 2), (300, 40_000, 2), (1100, 20_000, 2), (600, 10_000, 1), (3000, 1000, 1)]
 
 
@@ -200,7 +199,7 @@ STORE_ROUNDING_SHAPES = [(80, 100_000, 2), (300, 40_000, 2), (1100, 20_000, 2), 
 def test_float32_store_rounding_many_rows(batch: int, n: int, levels: int) -> None:
     # The same near-collinear data over many rows: with 256 rows or more the last merge launch's
     # workgroups (256 and 64 threads here, one a row) make their rows' hulls convex in the stored
-    # values themselves, and so do the span kernel's waves where they make the final hulls; with
+    # values themselves, and so do the groups' exact tests where a row is one group; with
     # fewer rows of two levels, the check and repair launches do.
     say(f"float32 store rounding: {batch} weighted near-collinear rows of {n}")
     rng = np.random.default_rng(11)

@@ -12,7 +12,7 @@ from gpu_util import check_fit, gpu_fit, tolerance
 
 pytestmark = pytest.mark.gpu
 
-# Rows over 32 elements take the span kernel and the merges; the expansion and the backward work
+# Rows over 32 elements take the group (or span) kernel and the merges; the expansion and the backward work
 # in tiles of 4096 elements unweighted, 2048 weighted, so these shapes cross their edges.
 SHAPES = [33, 63, 64, 65, 100, 255, 256, 511, 1000, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096]
 LONG_SHAPES = [4097, 8193, 20_000, 100_000]
@@ -98,7 +98,7 @@ def test_exact_ties_partition(n: int) -> None:
 
 @pytest.mark.parametrize("n", [100, 500, 3000])
 def test_nan_rows_long(n: int) -> None:
-    # (rows of 100 and 500: several rows a wave of the span kernel, NaN rows among them)
+    # (rows of one group each, NaN rows among them)
     rng = np.random.default_rng(1)
     y = rng.standard_normal((40, n))
     y[3, 17] = np.nan
@@ -411,8 +411,8 @@ def test_many_rows_of_one_span(batch: int, n: int) -> None:
 
 @pytest.mark.parametrize(("batch", "n"), [(9_000, 100), (8_192, 256), (2_000, 512), (3_000, 1000), (5_000, 1500)])
 def test_several_rows_a_wave(batch: int, n: int) -> None:
-    # rows of at most 2048 elements: several rows a wave of the span kernel, a power-of-two
-    # number of spans each, merged per row in the wave
+    # rows of at most 2048 elements: one small workgroup a row, or one row a lane of the span
+    # kernel
     print(f"rows a wave batch={batch} n={n}", flush=True)
     check_many_rows(batch, n)
 
@@ -583,9 +583,8 @@ def chord_rows(rows: int, n: int, dtype: type, weighted: bool, seed: int) -> tup
 @pytest.mark.parametrize("weighted", [False, True])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_candidate_filter_same_bits(dtype: type, weighted: bool, increasing: bool) -> None:
-    # A grid of at most two waves a SIMD (600 rows of 5000: 600 waves) runs the span kernel's
-    # stronger candidate test, which drops points lying clearly above the chord of their
-    # neighbours two elements away; 3000 rows (3000 waves, the same spans of 80) run without it. The same rows through
+    # Small and large batches of rows of one group (600 and 3000 rows of 5000), whose points clearly
+    # above a chord drop before the exact tests. The same rows in
     # both give the same bits, and the oracle's fit (and, but for the rows over 24 decades, whose
     # sums round differently in any order, its partition).
     from torchisotonic_amd import _ext

@@ -190,7 +190,7 @@ int fwd_impl(const void* y, const void* w, void* out, uint32_t* starts, uint32_t
     if (int rc = launched(hipGetLastError(), "weight check")) return rc;
     if (weights_read != nullptr)
       if (int rc = launched(hipEventRecord(weights_read, hs), "weights-read event")) return rc;
-    // (rows over 32 elements: the span kernel's first thread stores the mark as it starts, one
+    // (rows over 32 elements: the fit's first kernel's first thread stores the mark as it starts, one
     // launch fewer)
     if (weights_mark != nullptr && n > ti::kShortMax) start_mark = weights_mark;
     else if (weights_mark != nullptr)
@@ -211,7 +211,7 @@ int fwd_impl(const void* y, const void* w, void* out, uint32_t* starts, uint32_t
   if ((reinterpret_cast<uintptr_t>(workspace) & 255) != 0) return fail(TI_EINVAL, "workspace must be 256-byte aligned");
   if (batch * plan.tiles_per_row > 0x7FFFFFFF) return fail(TI_ESIZE, "too many tiles");
   ti::TileArgs a{y, w, out, starts, bad_weight, batch, n, dtype, flags, y_min, y_max, hs};
-  a.weights_read = weights_read;  // after the span kernel, the first of several
+  a.weights_read = weights_read;  // after the first kernel of several
   a.weights_mark = weights_mark;  // likewise
   a.start_mark = start_mark;
   a.mark_value = mark_value;

@@ -1,5 +1,5 @@
-// The expansion of one row's final hull by the workgroup that made it (the span kernel's wave
-// for rows of one merge level, the last merge launch's workgroup for rows of several): the
+// The expansion of one row's final hull by the workgroup that made it (the group
+// kernel's for rows of one group, the last merge launch's for rows of several): the
 // row's tile records, start bits and fit, in place of the rank and expansion launches.
 #pragma once
 

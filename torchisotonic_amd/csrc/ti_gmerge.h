@@ -1,5 +1,5 @@
 // The merge of child hulls in the parent's global array (merge_global), shared by the merge
-// kernel and the span kernel's group merge, with the vertex accessors and the bridge it uses.
+// kernel and the overflow kernel, with the vertex accessors and the bridge it uses.
 #pragma once
 
 #include "ti_common.h"

@@ -30,8 +30,6 @@ namespace ti {
 
 namespace {
 
-
-
 // Float32 data keeps its hull sums rounded to float64 in the vertex store (NodeOut). Rounded one
 // by one, a hull that the double-double merges found convex can turn slightly non-convex in the
 // stored values where points are nearly collinear, and the fit (its slopes) would step down
@@ -613,23 +611,21 @@ __global__ __launch_bounds__(256) void expand_kernel(ExpandArgs a) {
   }
 }
 
-// Rows of at most 2048 elements (one tile) in place of rank_kernel and expand_kernel, whose
-// one-tile-a-row layout leaves most threads of a workgroup idle on such rows: whole rows packed
-// into a workgroup of 256 threads, E consecutive elements a thread (E = 4 for rows up to 1024
-// elements, 8 up to 2048). Per row (one lane each): its record, as rank_kernel forms it for a
-// row of one tile, and its edge count; per edge: its fit (the slope rounded once, then clamped,
-// as expand_kernel forms it), its first element and that element's start bit, in LDS; per
-// element: its edge (a binary search for a thread's first element, then at most one step per
-// element). A NaN row is one edge, fit NaN.
-constexpr int kXpackMaxN = 2048;
-
+// Rows fitted one a lane (at most kSpanMax elements: LongPlan::levels == 0) in place of
+// rank_kernel and expand_kernel, whose one-tile-a-row layout leaves most threads of a workgroup
+// idle on such rows: whole rows packed into a workgroup of 256 threads, E consecutive elements a
+// thread. Per row (one lane each): its record, as rank_kernel forms it for a row of one tile, and
+// its edge count; per edge: its fit (the slope rounded once, then clamped, as expand_kernel forms
+// it), its first element and that element's start bit, in LDS; per element: its edge (a binary
+// search for a thread's first element, then at most one step per element). A NaN row is one edge,
+// fit NaN.
 template <typename T, bool W, int E, bool MAP = false>
 __global__ __launch_bounds__(256) void xpack_kernel(ExpandArgs a, TileRec* tiles, int rows_per_wg) {
   constexpr int NE = 256 * E;                  // elements a workgroup
   constexpr int NR = NE / (kShortMax + 1);     // rows a workgroup (n > 32)
   static_assert(NR <= kWave, "one lane per row");
   __shared__ T sl[NE];                         // per edge of the workgroup's rows: the fit
-  __shared__ int16_t est[NE];                  // per edge: its first element within its row (< 2048)
+  __shared__ int16_t est[NE];                  // per edge: its first element within its row (<= kSpanMax)
   __shared__ int roff[NR + 1];                 // per row: its first edge; [rows]: the edges in all
   __shared__ uint8_t rbad[NR];
   __shared__ uint32_t sbits[NE / 32 + NR];     // the rows' start-bit words, in order
@@ -939,7 +935,7 @@ LongPlan long_plan(int64_t batch, int64_t n, bool weighted, bool lo) {
   p.levels = level;  // merge launches; the final hulls are at level p.levels
   // the level whose vertex counts bound the final hulls' for a caller keeping them (ti_keep): two
   // below the final level (its merges, and then the expansion, overlap that caller's wait and
-  // allocation), but not level 0, whose counts the span kernel's fused merge overwrites
+  // allocation), but not level 0, which only overflowing groups write
   p.keep_level = p.levels <= 1 ? p.levels : std::max(1, p.levels - 2);
   p.slots = batch * p.npr[0] * (span0 + 1);
   bool any_defer = false, alt = false;
@@ -1152,8 +1148,8 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     if (e != hipSuccess) return e;
   }
   if (expanded) return hipSuccess;
-  if (t.n <= kXpackMaxN) {
-    // rows of one tile: records and fit together, whole rows a workgroup
+  if (p.levels == 0) {
+    // rows one a lane (at most kSpanMax elements): records and fit together, whole rows a workgroup
     ExpandArgs x;
     x.hulls = fin;
     x.batch = t.batch;
@@ -1167,27 +1163,24 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
     x.hi = t.hi;
     x.map = t.map;
     TileRec* recs = reinterpret_cast<TileRec*>(base + p.off_rank);
-    auto go = [&](auto E_) {
-      constexpr int E = decltype(E_)::value;
-      const int rpw = 256 * E / static_cast<int>(t.n);
-      const dim3 grid(static_cast<unsigned>((t.batch + rpw - 1) / rpw));
-      if (t.dtype == TI_F32) {
-        // (ragged rows of a block: float32 only)
-        if (t.map.rows != nullptr) {
-          if (W) xpack_kernel<float, true, E, true><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
-          else xpack_kernel<float, false, E, true><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
-        } else if (W) {
-          xpack_kernel<float, true, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
-        } else {
-          xpack_kernel<float, false, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
-        }
+    constexpr int E = 4;
+    const int rpw = 256 * E / static_cast<int>(t.n);
+    const dim3 grid(static_cast<unsigned>((t.batch + rpw - 1) / rpw));
+    if (t.dtype == TI_F32) {
+      // (ragged rows of a block: float32 only)
+      if (t.map.rows != nullptr) {
+        if (W) xpack_kernel<float, true, E, true><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
+        else xpack_kernel<float, false, E, true><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
+      } else if (W) {
+        xpack_kernel<float, true, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
       } else {
-        if (W) xpack_kernel<double, true, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
-        else xpack_kernel<double, false, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
+        xpack_kernel<float, false, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
       }
-      return hipGetLastError();
-    };
-    return t.n <= 1024 ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 8>{});
+    } else {
+      if (W) xpack_kernel<double, true, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
+      else xpack_kernel<double, false, E><<<grid, dim3(256), 0, t.stream>>>(x, recs, rpw);
+    }
+    return hipGetLastError();
   }
   {
     const int64_t tiles = t.batch * p.tiles_per_row;

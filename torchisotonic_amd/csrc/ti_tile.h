@@ -66,11 +66,11 @@ struct TileArgs {
   hipEvent_t weights_read = nullptr;  // recorded once every weight has been read, if given
   // Where given: mark_value written to *weights_mark (a word of host memory that the host polls)
   // once every weight has been read, with no event between kernels: at the start of the first
-  // merge launch after the span kernel, or by a kernel of one thread where none follows it
+  // merge launch after the group kernel, or by a kernel of one thread where none follows it
   uint32_t* weights_mark = nullptr;
   uint32_t mark_value = 0;
   // Where given (the weights read by a kernel before the fit): mark_value written to *start_mark
-  // by the span kernel's first thread as it starts, all of that kernel's reads being done
+  // by the first thread of the fit's first kernel as it starts, all of the earlier kernel's reads being done
   uint32_t* start_mark = nullptr;
   // Where given (rows over 32 elements): a bound on the final hulls' vertex counts (at least the
   // largest, at most n + 1) is written here (a device-visible word) and hulls_ready recorded once
@@ -392,7 +392,7 @@ struct ExpandArgs {
 struct LongPlan {
   int64_t tiles_per_row;  // expansion (and backward) tiles
   int64_t span0;          // elements per span (the first node level)
-  int rows_per_wave;      // > 1: the span kernel's wave holds that many short rows, 64 / it lanes each
+  int rows_per_wave;      // > 1: rows of at most 2048 elements whose store is laid out in 64 / it spans each
   int levels;
   int keep_level;  // the level whose vertex counts bound the final hulls' (see long_fit)
   int64_t batch;
