@@ -172,8 +172,8 @@ __device__ __forceinline__ void merge_chords(MergeChords& mc, int nch, DD es, DD
 // written then). A vertex's height over the chord is formed from its sums in the parent's frame
 // rounded to float64, with a margin of 2^-44 of all that goes into it.
 //
-// What bounds it: latency, three round trips to memory and about five rounds of tests, 4-12 us a
-// level; merging neighbouring hulls pairwise in six rounds of walks took 37-45 us (one row of 1e8:
+// What bounds it: latency, three round trips to memory and about five rounds of tests, 16-20 us a
+// level of one row of 1e8; merging neighbouring hulls pairwise in six rounds of walks took 37-45 us (one row of 1e8:
 // 36 + 45 + 11 us for its three levels).
 template <bool W, bool PR, int NT>
 __device__ bool merge_lds(const MergeArgs& a, const MergeSmall& sm, MergeChords& mc, const Points<W, PR, int>& v,
