@@ -213,6 +213,36 @@ def test_float32_store_rounding_many_rows(batch: int, n: int, levels: int) -> No
     assert float(np.abs(got - want).max()) <= tolerance(y)
 
 
+def chunk_joint_rows(kind: str) -> tuple[np.ndarray, np.ndarray]:
+    # Weighted float32 rows of one group that keep more points than its workgroup's LDS holds, so
+    # that chunks of 1920 ("steep") or 1280 elements are built one by one and merged: a point where
+    # two chunks meet is in both of them.
+    rng = np.random.default_rng(17)
+    if kind == "steep":  # a steep convex chain that ends where a chunk does, then a shallow one
+        i = np.arange(3840, dtype=np.float64)
+        y = np.where(i < 1920, -100 * np.abs((1919.5 - i) / 384) ** 6, 1e-12 * (i - 1919.5))
+        y = np.where(i < 1536, 1e-3 * i, y)
+        y = np.tile(y.astype(np.float32), (600, 1))
+        return y, (rng.random(y.shape) + 0.1).astype(np.float32)
+    i = np.arange(10_000, dtype=np.float64)
+    y = np.tile((1 + 1.2e-7 * i).astype(np.float32), (200, 1))
+    return y, (10.0 ** rng.uniform(-10, 0, y.shape)).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["steep", "wide weights"])
+def test_float32_chunk_joints_keep_the_fit_monotone(kind: str) -> None:
+    say(f"float32 chunk joints: {kind}")
+    y, w = chunk_joint_rows(kind)
+    assert _ext.geometry(*y.shape, True)["levels"] == 1
+    got, _ = gpu_fit(y, w)
+    assert (np.diff(got, axis=1) >= 0).all()
+    want, _ = oracle.pava(y.astype(np.float64), w.astype(np.float64))
+    # (a stored sum is rounded once, by 2^-53 of at most sum(w) max|y|; a slope takes two of them,
+    # and two weights', over an element's weight at least)
+    rounding = 2.0**-51 * float(w.astype(np.float64).sum(axis=1).max()) / float(w.min()) * float(np.abs(y).max())
+    assert float(np.abs(got - want).max()) <= tolerance(y) + rounding
+
+
 @pytest.mark.parametrize(("batch", "n"), [(1, 4_000_000), (300, 40_000), (600, 10_000), (3000, 1000), (9000, 100)])
 def test_float32_repair_chain_gives_the_same_hulls(batch: int, n: int) -> None:
     # The repair finishes a row with a sequential monotone chain after a cascade of removals

@@ -177,11 +177,14 @@ __device__ int chain_row(const VArr& v, int cnt, VPt* tile) {
   return top;
 }
 
+// LDS repair_row takes with NT threads (carved from a kernel's slots once they are free).
+constexpr size_t repair_lds_bytes(int nt) { return (nt + 2) * sizeof(VPt) + (nt / kWave + 1) * sizeof(int); }
+
 // A workgroup of NT threads removes, pass after pass, every vertex of the row's hull `o` on or
 // above the chord between its neighbours, until none is (the first pass is the check); after
 // `passes` removal passes the row is finished by chain_row. LDS: tile[NT + 2], wcount[NT / 64],
 // any.
-template <bool W, int NT>
+template <bool W, int NT, int B = 4>
 __device__ void repair_row(const NodeOut& o, VPt* tile, int* wcount, int& any, int passes) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const VArr v = dvarr_of(o);
@@ -190,20 +193,20 @@ __device__ void repair_row(const NodeOut& o, VPt* tile, int* wcount, int& any, i
   for (int pass = 0; pass <= passes; ++pass) {
     if (tid == 0) any = 0;
     __syncthreads();
-    // (four vertices a thread at a time, all their reads in flight together: a row's hull can
+    // (B vertices a thread at a time, all their reads in flight together: a row's hull can
     // have as many vertices as elements)
     bool found = false;
-    for (int i0 = 1 + tid; i0 < cnt - 1; i0 += 4 * NT) {
-      VPt a[4], b[4], c[4];
+    for (int i0 = 1 + tid; i0 < cnt - 1; i0 += B * NT) {
+      VPt a[B], b[B], c[B];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < B; ++u) {
         const int i = min(i0 + u * NT, cnt - 2);
         a[u] = vload<W>(v, i - 1);
         b[u] = vload<W>(v, i);
         c[u] = vload<W>(v, i + 1);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) found |= vpools<W>(a[u], b[u], c[u]);
+      for (int u = 0; u < B; ++u) found |= vpools<W>(a[u], b[u], c[u]);
     }
     if (__any(found) && lane == 0) any = 1;
     __syncthreads();

@@ -61,6 +61,7 @@ struct GroupArgs {
   NodeLevel spans;  // level 0
   NodeLevel out;    // the groups' level
   bool expand;      // rows of one group: the workgroup expands its row
+  int repair_passes;  // (overflow_kernel, such rows of float32 data) see repair_row
   RowExpand xp;
   RowMap map;
   uint32_t* mark;   // (where given) mark_value stored to *mark by the kernel's first thread
@@ -663,15 +664,22 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
       uint32_t bits = 0;
 #pragma unroll
       for (int k = 0; k < E; ++k) bits |= y[k] < (k + 1 < E ? y[k + 1 < E ? k + 1 : 0] : ynext) ? 1u << k : 0u;
-      const int t0 = tid * E, inner = max(0, min(E, clen - 1 - t0)), jend = clen - 1 - t0;
+      const int t0 = tid * E, inner = max(0, min(E, clen - 1 - t0));
       bits &= (1u << inner) - 1u;
-      if (jend >= 0 && jend < E) bits |= 1u << jend;
       int all;
       int pos = place<NT>(__popc(bits) + (tid == 0 ? 1 : 0), all, sh);
+      // the chunk's ends, from the sums that its neighbours' ends come from: a point where two
+      // chunks meet is one point, to its last bit (summed otherwise in each, 34 of 600 weighted
+      // rows of 3840 stepped down)
       if (tid == 0) {
         // (float32: the pair's sum, rounded once)
-        pput(pts, pos++, PR ? HPt{p0, cs.hi, cs.lo, cw.hi, cw.lo} : HPt{p0, cs.hi + cs.lo, 0.0, cw.hi + cw.lo, 0.0});
+        const auto end = [](int i, DD s, DD w) {
+          return PR ? HPt{i, s.hi, s.lo, w.hi, w.lo} : HPt{i, s.hi + s.lo, 0.0, w.hi + w.lo, 0.0};
+        };
+        pput(pts, pos++, end(p0, cs, cw));
+        pput(pts, all, end(p0 + clen, es, ew));
       }
+      ++all;
       emit<T, W, E>(pts, pos, bits, p0 + t0, false, b, y, w);
       cs = uniform_dd(es);
       if constexpr (W) cw = uniform_dd(ew);
@@ -701,6 +709,26 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
     ma.child_elems = 0;
     merge_global<W, true, NT>(ma, sm, mr.rlo, mr.rhi, mr.pre, g.row, c0, nch, out);
     __syncthreads();
+    // A row's final hull of float32 data convex in its stored values: the chunks' hulls are, and
+    // share their points, but a bridge found by a search over nearly collinear points can miss by
+    // their rounding. A triple that holds vertices of two chunks is tested; where one fails, the
+    // whole hull is. (Longer rows: their hulls, after the last merge.)
+    if constexpr (!PR) {
+      if (a.expand) {
+        const VArr v = dvarr_of(out);
+        bool dented = false;
+        for (int c = 1 + tid; c < nch; c += NT) {
+          for (int k = max(mr.pre[c] - 1, 1); k <= min(mr.pre[c], sm.total - 2); ++k)
+            dented |= vpools<W>(vload<W>(v, k - 1), vload<W>(v, k), vload<W>(v, k + 1));
+        }
+        if (__syncthreads_or(dented)) {
+          VPt* tile = reinterpret_cast<VPt*>(region);
+          int* wcount = reinterpret_cast<int*>(tile + NT + 2);
+          repair_row<W, NT, 1>(out, tile, wcount, wcount[NT / kWave], a.repair_passes);
+          __syncthreads();
+        }
+      }
+    }
     if constexpr (MAP) {
       // (the pad's block: see group_kernel)
       if (g.len > len) {
@@ -745,7 +773,7 @@ hipError_t overflow_launch(GroupArgs a, hipStream_t stream) {
   a.cap = (a.chunk * a.span0 + 1 + 3) & ~3;
   int region = std::max(a.cap * point_bytes<W, PR, uint16_t>(), (NT * E + NT) * tb);
   region = std::max(region, static_cast<int>(((sizeof(MergeSmall) + 63) & ~size_t(63)) + sizeof(MergeRanges)));
-  if (a.expand) region = std::max(region, expand_lds_min(a.g_elems, NT, tb));
+  if (a.expand) region = std::max({region, expand_lds_min(a.g_elems, NT, tb), static_cast<int>(repair_lds_bytes(NT))});
   region = (region + 63) & ~63;
   a.xp.lds_bytes = region;
   return launch_lds(overflow_kernel<T, W, NT, E, MAP>, a, std::min<int64_t>(a.batch * a.gpr, 2048), NT,
@@ -798,7 +826,7 @@ hipError_t group_shape(const GroupArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t group_run(const TileArgs& t, const NodeLevel& spans, int64_t span0, const NodeLevel& out, int64_t g_elems,
-                     TileRec* tiles) {
+                     TileRec* tiles, int repair_passes) {
   GroupArgs a{};
   a.y = t.y;
   a.w = t.w;
@@ -812,6 +840,7 @@ hipError_t group_run(const TileArgs& t, const NodeLevel& spans, int64_t span0, c
   a.spans = spans;
   a.out = out;
   a.expand = tiles != nullptr;
+  a.repair_passes = repair_passes;
   a.xp.n = t.n;
   a.xp.out = t.out;
   a.xp.starts = t.starts;

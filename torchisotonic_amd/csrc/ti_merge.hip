@@ -244,9 +244,6 @@ __device__ bool merge_lds(const MergeArgs& a, const MergeSmall& sm, MergeChords&
 // Rows enough for their final merge workgroups to read their hulls at the GPU's bandwidth.
 constexpr bool batch_fills_gpu(int64_t batch) { return batch >= 256; }
 
-// LDS repair_row takes with NT threads (carved from a merge kernel's slots once they are free).
-constexpr size_t repair_lds_bytes(int nt) { return (nt + 2) * sizeof(VPt) + (nt / kWave + 1) * sizeof(int); }
-
 // One workgroup of NT threads per parent node: kGroup children (fewer at a row's end) -> the
 // parent's hull. NT grows where few parents share the GPU (the upper levels), so that their
 // larger hulls still take few slots per thread.
@@ -1001,18 +998,19 @@ hipError_t long_fit(const TileArgs& t, const LongPlan& p, void* ws) {
   // Rows of one span: their hulls from span_run, one row a lane. Longer rows: level 1, the groups'
   // hulls, from group_run, which also expands rows of one group (their tile records, start bits
   // and fit), so nothing follows it.
-  // Float32 data: the final hulls convex in their stored values. A span's or a group's hull is
-  // built on those values; a final level of two or more has a merge workgroup for every row,
-  // which repairs its hull at its end (fold) where rows are enough to spread those workgroups
-  // over the GPU (one workgroup reading a hull of millions of vertices would take milliseconds);
-  // otherwise two launches after the merges do.
+  // Float32 data: the final hulls convex in their stored values. A span's hull, and a group's
+  // where its candidates fit LDS, is built on those values; a group merged from its chunks' hulls
+  // is repaired by the workgroup that merged it; a final level of two or more has a merge
+  // workgroup for every row, which repairs its hull at its end (fold) where rows are enough to
+  // spread those workgroups over the GPU (one workgroup reading a hull of millions of vertices
+  // would take milliseconds); otherwise two launches after the merges do.
   const int repair_passes = (t.flags & TI_REPAIR_CHAIN) != 0 ? 0 : kRepairPasses;
   const bool fold = !p.lo && p.levels >= 2 && batch_fills_gpu(t.batch);
   TileRec* const recs_at = reinterpret_cast<TileRec*>(base + p.off_rank);
   const bool one_group = p.levels == 1;
   hipError_t e = p.levels == 0 ? span_run(t, p.level(ws, 0))
                                : group_run(t, p.level(ws, 0), p.span0, p.level(ws, 1),
-                                           one_group ? t.n : kGroup * p.span0, one_group ? recs_at : nullptr);
+                                           one_group ? t.n : kGroup * p.span0, one_group ? recs_at : nullptr, repair_passes);
   if (e != hipSuccess) return e;
   // every weight has been read (and the flag set if one is not positive)
   if (t.weights_read != nullptr && (e = hipEventRecord(t.weights_read, t.stream)) != hipSuccess) return e;

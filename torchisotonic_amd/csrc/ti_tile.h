@@ -438,9 +438,10 @@ hipError_t span_run(const TileArgs& t, const NodeLevel& hulls);
 // Level 1 (or the rows' final hulls) from groups of g_elems elements, one workgroup a group:
 // out's nodes, one a group; spans: level 0, in whose slots a group of too many candidates builds
 // its chunks' hulls. tiles given (rows of one group): the workgroup also writes its row's fit,
-// start bits and tile records.
+// start bits and tile records, a hull merged from chunks' having been made convex in its stored
+// values (float32; repair_passes removal passes before the chain).
 hipError_t group_run(const TileArgs& t, const NodeLevel& spans, int64_t span0, const NodeLevel& out, int64_t g_elems,
-                     TileRec* tiles);
+                     TileRec* tiles, int repair_passes);
 
 // Backward of long rows, from the forward's final hulls and tile ranks (its workspace).
 struct LongGradArgs {
