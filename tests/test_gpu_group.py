@@ -81,6 +81,34 @@ def test_margin_over_every_height(n: int) -> None:
         assert float(np.abs(got - want).max()) <= 4 * np.finfo(dtype).eps * 1e25
 
 
+@pytest.mark.parametrize("n", [200, 512, 2048, 3840, 5000, 16384, 33_000])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_sums_over_threads_carry_their_rounding(n: int, weighted: bool) -> None:
+    # Pairs 2^60, -2^60 on either side of a multiple of 32 (so never in one thread's elements, whose
+    # sum is a float64), the rest of their two threads' elements 0: each pair cancels exactly, and
+    # beside it the sums across threads keep the other elements' parts, nine orders under 2^60's
+    # last place, only with their rounding errors. Increasing rows pool a pair and its zeros; the
+    # fit elsewhere is that of the row with the pair put to 0.
+    rng = np.random.default_rng(n)
+    y = (np.linspace(-1, 1, n) + rng.standard_normal((4, n))).astype(np.float32)
+    for row in y:
+        for m in [m for m in rng.permutation(np.arange(1, n // 32)) if m % 64 != 0][: max(1, n // 256)]:
+            row[32 * m - 32:32 * m + 32] = 0
+    plain = y.copy()
+    for r, row in enumerate(y):
+        # (every second run of 64 zeros; none across groups, whose points are float64s from its start)
+        at = [m for m in range(1, n // 32) if m % 64 != 0 and not row[32 * m - 32:32 * m + 32].any()]
+        for m in at[::2]:
+            row[32 * m - 1], row[32 * m] = 2.0**60, -(2.0**60)
+    w = (rng.random(y.shape) + 0.1).astype(np.float32) if weighted else None
+    if weighted:
+        w[y != plain] = 1
+    got, _ = gpu_fit(y, w)
+    want, _ = oracle.pava(plain, w, acc="f64")
+    assert (y != plain).any()
+    assert float(np.abs(got - want).max()) <= 4 * 2.0**-23 * float(np.abs(plain).max())
+
+
 def test_ragged_rows_end_where_they_end() -> None:
     # rows read in place up to their own length, the block's rest one block of pad: lengths around
     # the shapes' edges in one bucket, and rising rows that overflow it

@@ -7,7 +7,7 @@
 // every point is dropped by one test against a chord that is known to lie under it:
 //
 //   1. each thread holds E consecutive elements in registers; their sums, scanned over the
-//      workgroup (double-double), place the threads' first points (the coarse points);
+//      workgroup with their rounding errors, place the threads' first points (the coarse points);
 //   2. a lower hull of the coarse points, roughly: per wave, a few rounds in which every point
 //      above a chord of two other points drops out, all at once, on a 64-bit mask of the lanes;
 //      then the same over the points that are left of all waves, at most 64 of them (more, on
@@ -251,10 +251,12 @@ struct RunSums {
   }
 };
 
-// The sums before the thread's first element: in its wave (x), and before the wave (b). Float32
-// data is summed within a wave in float64 (32 terms a thread at most, then six scan steps: less
-// rounding than one thread's sum of 256), float64 data in double-double (xs, xw from the group's
-// start); across waves both are double-double, and a point's sums are rounded once.
+// The sums before the thread's first element (x), and before its wave (b). A thread's own sums (32
+// elements at most) of float32 data are float64, of float64 data double-double; from there on,
+// across lanes and waves, both are pairs whose second part holds the first's rounding errors, and a
+// point's sums are rounded once at the end (float32) or not at all. Where values cancel (2^60 and
+// -2^60 beside ordinary ones) a plain float64 scan lost the rest: errors of up to six times the
+// largest other value.
 struct BaseSums {
   DD xs, xw, bs, bw;
 };
@@ -264,33 +266,41 @@ __device__ __forceinline__ double uniform_f64(double v) {
 }
 __device__ __forceinline__ DD uniform_dd(DD v) { return DD{uniform_f64(v.hi), uniform_f64(v.lo)}; }
 
+// (float32: the errors summed and the pair not renormalised, eight operations in place of eleven:
+// an error under 2^-104 of the terms' magnitudes either way)
 template <bool PR>
 __device__ __forceinline__ DD sums_plus(DD a, DD b) {
   if constexpr (PR) {
     return dd_add(a, b);
   } else {
-    const DD t = two_sum(a.hi, b.hi);  // (b a float64; the errors summed, the pair not renormalised)
-    return DD{t.hi, a.lo + t.lo};
+    const DD t = two_sum(a.hi, b.hi);
+    return DD{t.hi, t.lo + (a.lo + b.lo)};
   }
 }
+// x and a thread's sum after it.
 template <bool PR>
-__device__ __forceinline__ DD sums_point(DD b, DD x, double t, double tl) {
-  if constexpr (PR) return dd_add(x, DD{t, tl});
-  else return DD{b.hi + (b.lo + (x.hi + t)), 0.0};
+__device__ __forceinline__ DD sums_point(DD x, double t, double tl) {
+  if constexpr (PR) {
+    return dd_add(x, DD{t, tl});
+  } else {
+    const DD s = two_sum(x.hi, t);
+    return DD{s.hi + (s.lo + x.lo), 0.0};
+  }
 }
 
-// The lanes' sums (hi, lo) before each lane, and of the whole wave.
+// The lanes' sums (hi, lo) before each lane, and of the whole wave (see wave_incl_dd).
 template <bool PR>
 __device__ __forceinline__ void wave_scan(double hi, double lo, DD& before, DD& all) {
-  if constexpr (PR) {
-    const DD i = wave_incl_dd(DD{hi, lo});
-    before = wave_shr1_dd(i);
-    all = wave_last_dd(i);
-  } else {
-    const double i = wave_incl_f64(hi);
-    before = DD{dpp_f64<0x138, 0xF>(i), 0.0};
-    all = DD{wave_last_f64(i), 0.0};
-  }
+  DD v{hi, lo};
+  if constexpr (PR) v = dd_add(dpp_dd<0x111, 0xF>(v), v);
+  else v = two_sum(dpp_f64<0x111, 0xF>(hi), hi);  // (lo is zero)
+  v = sums_plus<PR>(dpp_dd<0x112, 0xF>(v), v);
+  v = sums_plus<PR>(dpp_dd<0x114, 0xF>(v), v);
+  v = sums_plus<PR>(dpp_dd<0x118, 0xF>(v), v);
+  v = sums_plus<PR>(dpp_dd<0x142, 0xA>(v), v);
+  v = sums_plus<PR>(dpp_dd<0x143, 0xC>(v), v);
+  before = wave_shr1_dd(v);
+  all = wave_last_dd(v);
 }
 
 // The points of `mine` (bit k: the point after element k) to slots pos, pos + 1, ...
@@ -306,8 +316,8 @@ __device__ __forceinline__ void emit(const GPoints<W, sizeof(T) == 8>& pts, int 
     if ((mine >> k) & 1) {
       HPt p;
       p.i = t0 + k + 1;
-      const DD S = bad ? DD{0.0, 0.0} : sums_point<PR>(b.bs, b.xs, t.s, t.sl);
-      const DD Wd = W ? sums_point<PR>(b.bw, b.xw, t.w, t.wl) : DD{0.0, 0.0};
+      const DD S = bad ? DD{0.0, 0.0} : sums_point<PR>(b.xs, t.s, t.sl);
+      const DD Wd = W ? sums_point<PR>(b.xw, t.w, t.wl) : DD{0.0, 0.0};
       p.s = S.hi;
       p.sl = S.lo;
       p.w = Wd.hi;
@@ -424,14 +434,12 @@ __device__ __forceinline__ GroupSums group_sums(const GroupArgs& a, const GroupT
   }
   r.maxabs = uniform_f64(r.maxabs);
   r.bad = __builtin_amdgcn_readfirstlane(r.bad ? 1 : 0) != 0;
-  if constexpr (PR) {
-    r.b.xs = dd_add(r.b.bs, r.b.xs);
-    if constexpr (W) r.b.xw = dd_add(r.b.bw, r.b.xw);
-  }
+  r.b.xs = sums_plus<PR>(r.b.bs, r.b.xs);
+  if constexpr (W) r.b.xw = sums_plus<PR>(r.b.bw, r.b.xw);
   if (threadIdx.x == nt - 1) {  // (the last wave's: every element is in its sums)
     const int pad = g.len - g.glen;  // (ragged rows: the pad, of weight 1)
-    const DD S = r.bad ? DD{0.0, 0.0} : sums_plus<PR>(r.b.bs, r.wave_s);
-    const DD Wd = W ? sums_plus<PR>(r.b.bw, r.wave_w) : DD{static_cast<double>(g.glen), 0.0};
+    const DD S = r.bad ? DD{0.0, 0.0} : dd_add(r.b.bs, r.wave_s);
+    const DD Wd = W ? dd_add(r.b.bw, r.wave_w) : DD{static_cast<double>(g.glen), 0.0};
     const DD Sp = MAP && !r.bad ? dd_add(S, pad * signed_pad(a)) : S;
     const DD Wp = MAP ? dd_add(Wd, static_cast<double>(pad)) : Wd;
     *out.bad = r.bad ? 1 : 0;
@@ -470,8 +478,7 @@ __global__ __launch_bounds__(NT, 4) void group_kernel(GroupArgs a) {
   g.load_at(a, 0, len, region + wave * (kWave * E * static_cast<int>(sizeof(T))), y, w);
   const GroupSums q = group_sums(a, g, sh, out, y, w, nt);
   const BaseSums& b = q.b;
-  const CPt me{sums_point<PR>(b.bs, b.xs, 0.0, 0.0).hi,
-               W ? sums_point<PR>(b.bw, b.xw, 0.0, 0.0).hi : static_cast<double>(min(t0, len))};
+  const CPt me{b.xs.hi, W ? b.xw.hi : static_cast<double>(min(t0, len))};
   opaque(y);
   if constexpr (W) opaque(w);
 
@@ -656,10 +663,8 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
         es = sums_plus<PR>(es, DD{sh.tot[2][q], sh.tot[3][q]});
         if constexpr (W) ew = sums_plus<PR>(ew, DD{sh.tot[0][q], sh.tot[1][q]});
       }
-      if constexpr (PR) {
-        b.xs = dd_add(b.bs, b.xs);
-        if constexpr (W) b.xw = dd_add(b.bw, b.xw);
-      }
+      b.xs = sums_plus<PR>(b.bs, b.xs);
+      if constexpr (W) b.xw = sums_plus<PR>(b.bw, b.xw);
       const T ynext = fy[min(tid + 1, NT - 1)];
       uint32_t bits = 0;
 #pragma unroll
