@@ -81,6 +81,30 @@ def test_margin_over_every_height(n: int) -> None:
         assert float(np.abs(got - want).max()) <= 4 * np.finfo(dtype).eps * 1e25
 
 
+@pytest.mark.parametrize(("n", "batches"), [(1100, (4, 3000)), (2001, (4, 3000)), (2500, (4, 132, 600)),
+                                            (9001, (4, 40, 72, 132, 600)), (16384, (4, 20, 260)), (33_000, (4, 100))])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_overflowing_groups_shared_by_workgroups(n: int, batches: tuple[int, ...], dtype: type) -> None:
+    # A group of more candidates than slots is built by one workgroup or, where groups are few, by
+    # several that share its chunks: as many as chunks for 4 rows, two or three of them for up to 128
+    # groups, one from 256 on. The same rows give the same bits whoever builds them, and the oracle's.
+    print(f"overflowing groups n={n} {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(n)
+    y = np.stack([rows(k, n, rng) for k in ("rise", "drops", "noise", "rise")]).astype(dtype)
+    w = (rng.random(y.shape) + 0.1).astype(dtype)
+    for ww in (None, w):
+        first = None
+        for b in batches:
+            if _ext.geometry(b, n, ww is not None) != _ext.geometry(4, n, ww is not None):
+                first = None  # (other groups: compared with the oracle only)
+            got, starts = check_fit(np.tile(y, (b // 4, 1)), None if ww is None else np.tile(ww, (b // 4, 1)))
+            assert (np.diff(got, axis=1) >= 0).all()
+            if first is None:
+                first = got[:4], starts[:4]
+            np.testing.assert_array_equal(got, np.tile(first[0], (b // 4, 1)))
+            np.testing.assert_array_equal(starts, np.tile(first[1], (b // 4, 1)))
+
+
 @pytest.mark.parametrize("n", [200, 512, 2048, 3840, 5000, 16384, 33_000])
 @pytest.mark.parametrize("weighted", [False, True])
 def test_sums_over_threads_carry_their_rounding(n: int, weighted: bool) -> None:

@@ -55,7 +55,10 @@ struct GroupArgs {
   int span0;        // elements per span of level 0 (a chunk's hull lies in its spans' slots)
   int nt;           // group_kernel's threads
   int cap;          // point slots in LDS
-  int chunk;        // (overflow_kernel) spans per chunk, a power of two
+  int chunk, cpg;   // (overflow_kernel) spans per chunk, chunks per group
+  int parts;        // and workgroups that share a group's
+  NodeLevel chunks;  // level 0, a chunk a node: its hull, and in tot the sums before it; a group's
+                     // first node's bad counts its parts done
   int expand_at;    // the expansion's LDS, from the region's start
   unsigned flags;
   NodeLevel spans;  // level 0
@@ -72,8 +75,7 @@ struct GroupArgs {
 template <bool W, bool PR>
 using GPoints = Points<W, PR, uint16_t>;
 
-// Per group: the waves' totals and flags, candidate counts, the coarse list, a chunked group's
-// hull counts.
+// Per group: the waves' totals and flags, candidate counts, the coarse list.
 template <int NW>
 struct GroupShared {
   double tot[4][NW];  // per wave: W hi, lo, S hi, lo
@@ -83,13 +85,12 @@ struct GroupShared {
   int count[NW];
   int wc[NW];
   int result;
-  int ccnt[kGroup];
   double ls[kWave + 1], lw[kWave + 1];
   double end[2];  // the group's end, its pad included: W and S
 };
 
 __host__ __device__ constexpr int group_head_bytes(int nw) {
-  return (nw * (5 * 8 + 4 * 4) + 8 + kGroup * 4 + 2 * (kWave + 2) * 8 + 63) & ~63;
+  return (nw * (5 * 8 + 4 * 4) + 8 + 2 * (kWave + 2) * 8 + 63) & ~63;
 }
 
 // E consecutive elements a thread from the wave's 64 * E: loaded in 16-byte pieces, each load
@@ -569,7 +570,20 @@ __global__ __launch_bounds__(NT, 4) void group_kernel(GroupArgs a) {
   int all;
   int pos = place<NT>(__popc(bits) + extra, all, sh, nt);
   if (all + 1 > a.cap) {
-    if (tid == 0) *out.count = kOverflow;
+    // (a chunk begins where a thread's elements do: see overflow_shape)
+    const int ce = a.chunk * a.span0;
+    const int64_t c0 = static_cast<int64_t>(g.grp) * a.cpg;
+    if (t0 < len && t0 % ce == 0) {
+      double* const tot = node_at(a.chunks, W, g.row, c0 + t0 / ce).tot;
+      tot[0] = W ? b.xw.hi : 0.0;
+      tot[1] = W ? b.xw.lo : 0.0;
+      tot[2] = b.xs.hi;
+      tot[3] = b.xs.lo;
+    }
+    if (tid == 0) {
+      *node_at(a.chunks, W, g.row, c0).bad = 0;
+      *out.count = kOverflow;
+    }
     return;
   }
   if (extra != 0) pput(pts, pos++, HPt{0, 0.0, 0.0, 0.0, 0.0});
@@ -602,10 +616,15 @@ __global__ __launch_bounds__(NT, 4) void group_kernel(GroupArgs a) {
 
 // The groups of more candidates than slots (kOverflow): the points at every rise, a chunk of spans
 // at a time, each chunk's hull to its spans' slots in the group's frame, then those merged by
-// reference (merge_global). A workgroup takes every gridDim.x-th group; where none overflowed
-// (noisy data) the launch is one read of the counts. (A kernel of its own: in group_kernel its
-// registers would halve every group's occupancy. Few threads a workgroup, as most of the merge
-// keeps a few busy, and up to eight workgroups a CU.)
+// reference (merge_global). A workgroup a group, or several, which share its chunks, where groups
+// are few. Where none overflowed (noisy data) the launch is one read of the counts. (A kernel of its own: in group_kernel its registers would
+// halve every group's occupancy. Few threads a workgroup, as most of the merge keeps a few busy,
+// and up to eight workgroups a CU.)
+//
+// What bounds it: a chunk's rounds and the merge's chains of reads. With a workgroup a group
+// whatever their number, and float64 in 128 threads of 8 elements: one rising row of 16384 166 us
+// (weighted float64 377), now 128 (154); 200 of them 203 (484), now 209 (289); 1000 weighted
+// float64 ones of 5000 317, now 253.
 template <typename T, bool W, int NT, int E, bool MAP>
 __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
   constexpr bool PR = sizeof(T) == 8;
@@ -614,28 +633,31 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
   GroupShared<NW>& sh = *reinterpret_cast<GroupShared<NW>*>(group_lds);
   char* const region = group_lds + group_head_bytes(NW);
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = wave_index();
-  const unsigned groups = static_cast<unsigned>(a.batch * a.gpr);
+  // (part p of a group's `parts`: chunks p, p + parts, ...)
+  const unsigned parts = static_cast<unsigned>(a.parts);
+  const unsigned items = static_cast<unsigned>(a.batch * a.gpr) * parts;
   const int* const counts = node_at(a.out, W, 0, 0).count;
   bool any = false;
-  for (unsigned g0 = blockIdx.x + gridDim.x * tid; g0 < groups; g0 += gridDim.x * NT) any |= counts[g0] == kOverflow;
+  for (unsigned k = blockIdx.x + gridDim.x * tid; k < items; k += gridDim.x * NT) any |= counts[k / parts] == kOverflow;
   if (!__syncthreads_or(any)) return;
   const int ce = a.chunk * a.span0;
-  NodeLevel in = a.spans;  // a chunk a node
-  in.npr = (a.spans.npr0 + a.chunk - 1) / a.chunk;
-  in.spn = a.chunk;
   const GPoints<W, PR> pts = points_carve<W, PR, uint16_t>(region, a.cap);
   char* const slab = region + wave * (kWave * E * static_cast<int>(sizeof(T)));
-  for (unsigned gi = blockIdx.x; gi < groups; gi += gridDim.x) {
-    if (counts[gi] != kOverflow) continue;  // (the same in every thread: written by no one but below)
+  for (unsigned item = blockIdx.x; item < items; item += gridDim.x) {
+    const unsigned gi = item / parts;
+    const int part = static_cast<int>(item - gi * parts);
+    // (the same in every thread: overwritten once all of the group's parts, this one too, are done)
+    if (counts[gi] != kOverflow) continue;
     const GroupThread<T, W, NT, E, MAP> g(a, gi);
-    const NodeOut out = node_at(a.out, W, g.row, g.grp);
     const int len = g.glen;
     const int nch = (len + ce - 1) / ce;
-    const int64_t c0 = static_cast<int64_t>(g.grp) * (kGroup / a.chunk);
-    DD cs{0.0, 0.0}, cw{0.0, 0.0};  // the sums before the chunk
-    for (int chunk = 0; chunk < nch; ++chunk) {
+    if (part >= nch) continue;  // (a group at its row's end)
+    const int64_t c0 = static_cast<int64_t>(g.grp) * a.cpg;
+    for (int chunk = part; chunk < nch; chunk += a.parts) {
       __syncthreads();  // (the points, counts and totals before read by every thread)
       const int p0 = chunk * ce, clen = min(ce, len - p0);
+      const double* const tot = node_at(a.chunks, W, g.row, c0 + chunk).tot;
+      const DD cs{tot[2], tot[3]}, cw{tot[0], tot[1]};  // the sums before the chunk
       T y[E], w[W ? E : 1];
       g.load_at(a, p0, clen, slab, y, w);
       RunSums<T, W> t;
@@ -654,14 +676,11 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
       T* const fy = reinterpret_cast<T*>(region + NW * (kWave * E * static_cast<int>(sizeof(T))));
       fy[tid] = y[0];
       __syncthreads();
-      DD es = cs, ew = cw;
-      for (int q = 0; q < NW; ++q) {
-        if (q == wave) {
-          b.bs = es;
-          b.bw = ew;
-        }
-        es = sums_plus<PR>(es, DD{sh.tot[2][q], sh.tot[3][q]});
-        if constexpr (W) ew = sums_plus<PR>(ew, DD{sh.tot[0][q], sh.tot[1][q]});
+      b.bs = cs;
+      b.bw = cw;
+      for (int q = 0; q < wave; ++q) {
+        b.bs = sums_plus<PR>(b.bs, DD{sh.tot[2][q], sh.tot[3][q]});
+        if constexpr (W) b.bw = sums_plus<PR>(b.bw, DD{sh.tot[0][q], sh.tot[1][q]});
       }
       b.xs = sums_plus<PR>(b.bs, b.xs);
       if constexpr (W) b.xw = sums_plus<PR>(b.bw, b.xw);
@@ -673,43 +692,57 @@ __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
       bits &= (1u << inner) - 1u;
       int all;
       int pos = place<NT>(__popc(bits) + (tid == 0 ? 1 : 0), all, sh);
-      // the chunk's ends, from the sums that its neighbours' ends come from: a point where two
-      // chunks meet is one point, to its last bit (summed otherwise in each, 34 of 600 weighted
-      // rows of 3840 stepped down)
-      if (tid == 0) {
-        // (float32: the pair's sum, rounded once)
-        const auto end = [](int i, DD s, DD w) {
-          return PR ? HPt{i, s.hi, s.lo, w.hi, w.lo} : HPt{i, s.hi + s.lo, 0.0, w.hi + w.lo, 0.0};
-        };
-        pput(pts, pos++, end(p0, cs, cw));
+      // The chunk's ends: where the next chunk begins, from that chunk's own sums, so that the point
+      // where two chunks meet is one point, to its last bit (summed otherwise in each, 34 of 600
+      // weighted rows of 3840 stepped down). (float32: the pair's sum, rounded once)
+      const auto end = [](int i, DD s, DD w) {
+        return PR ? HPt{i, s.hi, s.lo, w.hi, w.lo} : HPt{i, s.hi + s.lo, 0.0, w.hi + w.lo, 0.0};
+      };
+      if (tid == 0) pput(pts, pos++, end(p0, cs, cw));
+      if (tid == NT - 1) {
+        DD es = sums_plus<PR>(b.bs, wave_s), ew = W ? sums_plus<PR>(b.bw, wave_w) : DD{0.0, 0.0};
+        if (chunk + 1 < nch) {
+          const double* const next = tot + 4;  // (the next chunk's)
+          es = DD{next[2], next[3]};
+          ew = DD{next[0], next[1]};
+        }
         pput(pts, all, end(p0 + clen, es, ew));
       }
       ++all;
       emit<T, W, E>(pts, pos, bits, p0 + t0, false, b, y, w);
-      cs = uniform_dd(es);
-      if constexpr (W) cw = uniform_dd(ew);
       __syncthreads();
       const int cnt = prune_all<NT>(pts, all, sh.wc, &sh.result);
-      const NodeOut o = node_at(in, W, g.row, c0 + chunk);
+      const NodeOut o = node_at(a.chunks, W, g.row, c0 + chunk);
       for (int k = tid; k < cnt; k += NT) {
         const HPt p = pget(pts, k);
         o.idx[k] = p.i;
         put_dd(o.shi, o.slo, k, p.s, p.sl);
         if constexpr (W) put_dd(o.whi, o.wlo, k, p.w, p.wl);
       }
-      if (tid == 0) sh.ccnt[chunk] = cnt;
+      if (tid == 0) *o.count = cnt;
     }
+    // The last of the group's parts to be done merges the chunks' hulls: every part's stores are
+    // made visible to the device before it is counted, and read after the last one was.
     __syncthreads();
+    if (parts > 1) {
+      if (tid == 0)
+        sh.result = __hip_atomic_fetch_add(node_at(a.chunks, W, g.row, c0).bad, 1, __ATOMIC_ACQ_REL,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      if (sh.result != min(a.parts, nch) - 1) continue;
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    const NodeOut out = node_at(a.out, W, g.row, g.grp);
     MergeSmall& sm = *reinterpret_cast<MergeSmall*>(region);
     MergeRanges& mr = *reinterpret_cast<MergeRanges*>(region + ((sizeof(MergeSmall) + 63) & ~size_t(63)));
     for (int c = tid; c < nch; c += NT) {
-      sm.cnt[c] = sh.ccnt[c];
+      sm.cnt[c] = *node_at(a.chunks, W, g.row, c0 + c).count;
 #pragma unroll
       for (int i = 0; i < 4; ++i) sm.tot[i][c] = 0.0;  // (the chunks are in the group's frame)
     }
     __syncthreads();
     MergeArgs ma;
-    ma.in = in;
+    ma.in = a.chunks;
     ma.out = a.out;
     ma.child_elems = 0;
     merge_global<W, true, NT>(ma, sm, mr.rlo, mr.rhi, mr.pre, g.row, c0, nch, out);
@@ -765,23 +798,42 @@ hipError_t launch_lds(K k, const GroupArgs& a, int64_t blocks, int threads, int 
   return hipGetLastError();
 }
 
-// The groups that overflowed. Chunks of at most 2048 elements (float64: 1024), a row's points each.
+// Chunks of at most 2048 elements (float64: 1024, in as many threads: its merge keeps more of them
+// busy), a multiple of 8 spans (float64: 4) of a multiple of 4 elements each (float64 groups of up
+// to 2048 elements: of 8; float32 ones never overflow), so a chunk begins where one of
+// group_kernel's threads does, whose sums it starts from.
+template <typename T>
+constexpr int kOverflowThreads = 256;
+template <typename T>
+constexpr int kOverflowElems = sizeof(T) == 8 ? 4 : 8;
+template <typename T>
+void overflow_shape(GroupArgs& a) {
+  a.chunk = std::min(kGroup, kOverflowThreads<T> * kOverflowElems<T> / a.span0 & (sizeof(T) == 8 ? ~3 : ~7));
+  a.cpg = (a.g_elems + a.chunk * a.span0 - 1) / (a.chunk * a.span0);
+  a.chunks = a.spans;
+  a.chunks.npr = a.gpr * a.cpg;
+  a.chunks.spn = a.chunk;
+}
+
+// The groups that overflowed. Several workgroups share a group where that gives up to a workgroup a
+// CU; each is counted by an atomic that first writes its XCD's L2 back, which many groups cannot
+// afford (1000 rising rows of 10000, a workgroup a chunk: 1795 us, a workgroup a group 180).
+constexpr int64_t kOverflowShare = 256;
 template <typename T, bool W, bool MAP>
 hipError_t overflow_launch(GroupArgs a, hipStream_t stream) {
   constexpr bool PR = sizeof(T) == 8;
   constexpr int tb = static_cast<int>(sizeof(T));
-  constexpr int NT = PR ? 128 : 256, E = 8;
+  constexpr int NT = kOverflowThreads<T>, E = kOverflowElems<T>;
+  const int64_t groups = a.batch * a.gpr;
+  a.parts = static_cast<int>(std::min<int64_t>(a.cpg, std::max<int64_t>(1, kOverflowShare / groups)));
   a.mark = nullptr;
-  a.chunk = 1;
-  while (a.chunk < kGroup && 2 * a.chunk * a.span0 <= NT * E) a.chunk *= 2;
-  if (a.chunk * a.span0 > NT * E) return hipErrorInvalidConfiguration;
   a.cap = (a.chunk * a.span0 + 1 + 3) & ~3;
   int region = std::max(a.cap * point_bytes<W, PR, uint16_t>(), (NT * E + NT) * tb);
   region = std::max(region, static_cast<int>(((sizeof(MergeSmall) + 63) & ~size_t(63)) + sizeof(MergeRanges)));
   if (a.expand) region = std::max({region, expand_lds_min(a.g_elems, NT, tb), static_cast<int>(repair_lds_bytes(NT))});
   region = (region + 63) & ~63;
   a.xp.lds_bytes = region;
-  return launch_lds(overflow_kernel<T, W, NT, E, MAP>, a, std::min<int64_t>(a.batch * a.gpr, 2048), NT,
+  return launch_lds(overflow_kernel<T, W, NT, E, MAP>, a, std::min<int64_t>(groups * a.parts, 2048), NT,
                     group_head_bytes(NT / kWave) + region, stream);
 }
 
@@ -801,6 +853,7 @@ hipError_t group_launch(GroupArgs a, hipStream_t stream) {
   // and at least 1028: what lets two workgroups or more share a CU's LDS.
   constexpr int kMost = PR ? std::max(1028, G / 8 + 4) : G <= 2048 ? 2052 : G >= 16384 ? (W ? 3076 : 4100) : G / 4 + 4;
   a.cap = (std::min(a.g_elems + 3, kMost) + 3) & ~3;
+  overflow_shape<T>(a);
   a.expand_at = (a.cap * point_bytes<W, PR, uint16_t>() + 63) & ~63;
   const int words4 = (((a.g_elems + 31) / 32) + 3) & ~3;
   int region = std::max(P > 2 ? a.nt * E * tb : 0, NW * (kWave + 1) * 16 + NT * tb);

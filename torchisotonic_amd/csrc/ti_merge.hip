@@ -906,6 +906,8 @@ LongPlan long_plan(int64_t batch, int64_t n, bool weighted, bool lo) {
     while (k > kmin && !fits(k)) k >>= 1;
     if (k > 1 && fits(k) && ((n + k - 1) / k <= kSpanMin || batch * k >= (int64_t{1} << 17))) {
       span0 = (n + k - 1) / k;
+      // (whole pieces of 8 elements: where a chunk of an overflowing group can begin)
+      if (n > 1024) span0 = (span0 + 7) & ~int64_t{7};
       p.rows_per_wave = static_cast<int>(kGroup / k);
     }
   }
