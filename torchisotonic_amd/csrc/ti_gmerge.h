@@ -251,8 +251,7 @@ __device__ void repair_row(const NodeOut& o, VPt* tile, int* wcount, int& any, i
 struct MergeSmall {
   int cnt[kGroup], off[kGroup];
   double tot[4][kGroup + 1];  // child offsets (W hi, lo, S hi, lo); [nch]: the parent's total
-  int keep[kGroup / 2], from[kGroup / 2];
-  int total, bad, rounds_max;
+  int total, bad;
 };
 
 // Slot s of the children laid end to end (each child's first vertex is the previous child's
