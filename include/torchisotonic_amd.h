@@ -51,11 +51,11 @@ extern "C" {
    whose next kernels read other data (a backward): they then do not wait behind its write-back.
    The results are the same with or without it. */
 #define TI_STREAM_OUT 16u
-/* A test hook (ti_fwd and its variants, float32 rows over 32 elements): the repair that makes
-   each final hull convex in its stored float64 values skips its parallel removal passes and
-   finishes every row it repairs with its one-pass sequential monotone chain, the form it
-   otherwise takes only after a cascade of removals longer than its pass limit. The results are
-   the same with or without it. */
+/* A test hook (ti_fwd and its variants, float32 rows of two levels or more, and rows of one group
+   whose merged chunks' joints need it): the repair that makes a final hull convex in its stored
+   float64 values skips its parallel removal passes and finishes every row it repairs with its
+   one-pass sequential monotone chain, the form it otherwise takes only after a cascade of
+   removals longer than its pass limit. The results are the same with or without it. */
 #define TI_REPAIR_CHAIN 32u
 
 /* The ABI version this library was built with (TI_ABI_VERSION). */
@@ -72,11 +72,13 @@ int64_t ti_starts_words(int64_t batch, int64_t n);
  * merge levels have few parents (fewer than 256 rows of 1e6 elements, say) a second store. */
 int ti_fwd_workspace(int64_t batch, int64_t n, int dtype, int weighted, size_t* bytes);
 
-/* Diagnostic: the kernel geometry ti_fwd takes for rows of more than 32 elements - elements per
- * span of its first kernel (one lane builds each span's hull), the merge launches that follow
- * it, and the rows per wave of the first kernel (1: a wave holds spans of one row). Rows of at
- * most 32 elements report 0, 0, 0. No counterpart in the reference: tests use it to show which
- * geometry a case exercises. */
+/* Diagnostic: the geometry ti_fwd takes for rows of more than 32 elements - elements per span, the
+ * unit of the vertex store (a group, which one workgroup of the first kernel builds, is up to 64 of
+ * them); the levels of groups and merges above the spans (0: rows built one a lane; 1: one group a
+ * row); and, where a row of at most 2048 elements is laid out in fewer than 64 spans, 64 over their
+ * number (else 1; before their size is rounded), which no kernel reads. Rows of at most 32 elements
+ * report 0, 0, 0. No counterpart in the reference: tests use it to show which geometry a case
+ * exercises. */
 int ti_fwd_geometry(int64_t batch, int64_t n, int weighted, int64_t* span0, int* levels,
                     int* rows_per_wave);
 

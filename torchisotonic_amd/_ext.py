@@ -242,8 +242,8 @@ def _workspace_bytes(kind: str, batch: int, n: int, dtype: int, weighted: bool) 
 
 
 def geometry(batch: int, n: int, weighted: bool) -> dict:
-    """The long-row forward's kernel geometry for a problem set (a diagnostic): elements per
-    span of its first kernel, merge launches after it, rows per wave of the first kernel."""
+    """The long-row forward's geometry for a problem set (a diagnostic): elements per span, levels
+    of groups and merges above the spans, and a figure of the store's layout (ti_fwd_geometry)."""
     span0, levels, rpw = _i64(0), _int(0), _int(0)
     _check(
         load().ti_fwd_geometry(batch, n, int(weighted), ctypes.byref(span0), ctypes.byref(levels), ctypes.byref(rpw)),

@@ -850,7 +850,9 @@ hipError_t group_launch(GroupArgs a, hipStream_t stream) {
   a.nt = NT <= 2 * kWave ? NT : (a.g_elems + E * kWave - 1) / (E * kWave) * kWave;
   // Slots: every point of a group of up to 2048 elements (float64: half); beyond, one for every
   // four elements (noisy trends leave a candidate in eight or fewer), float64 one for every eight
-  // and at least 1028: what lets two workgroups or more share a CU's LDS.
+  // and at least 1028: what lets two workgroups or more share a CU's LDS. Weighted groups of over
+  // 8192: three for every sixteen (18 bytes a slot and 4 in the expansion's table: with 4100 one
+  // workgroup would take 94 KB of the CU's 160).
   constexpr int kMost = PR ? std::max(1028, G / 8 + 4) : G <= 2048 ? 2052 : G >= 16384 ? (W ? 3076 : 4100) : G / 4 + 4;
   a.cap = (std::min(a.g_elems + 3, kMost) + 3) & ~3;
   overflow_shape<T>(a);

@@ -125,8 +125,8 @@ __global__ __launch_bounds__(kRepairThreads) void repair_kernel(NodeLevel fin, u
   if (tid == 0) *o.count = cnt;
 }
 
-// Fewer slots go to the exact tests without chords (4000 rows of 16384 to 65536 elements, four
-// children of about 30 vertices each: the chords took 4 us of a 74 us launch).
+// Fewer slots go to the exact tests without chords (1000 rows of 65536 elements, four children of
+// about 30 vertices each: the chords took 4 us of a 74 us launch).
 constexpr int kChordSlots = 256;
 
 // The chord under each child's vertices (a point and the slope), from a rough hull of the
@@ -173,8 +173,8 @@ __device__ __forceinline__ void merge_chords(MergeChords& mc, int nch, DD es, DD
 // rounded to float64, with a margin of 2^-44 of all that goes into it.
 //
 // What bounds it: latency, three round trips to memory and about five rounds of tests, 16-20 us a
-// level of one row of 1e8; merging neighbouring hulls pairwise in six rounds of walks took 37-45 us (one row of 1e8:
-// 36 + 45 + 11 us for its three levels).
+// level of one row of 1e8; merging neighbouring hulls pairwise in six rounds of walks took 37-45 us
+// (one row of 1e8: 36 + 45 + 11 us for its three levels).
 template <bool W, bool PR, int NT>
 __device__ bool merge_lds(const MergeArgs& a, const MergeSmall& sm, MergeChords& mc, const Points<W, PR, int>& v,
                           int cap, int64_t row, int64_t c0, int nch, const NodeOut& pout) {

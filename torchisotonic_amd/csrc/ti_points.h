@@ -160,7 +160,9 @@ __device__ int prune(const Points<W, PR, I>& v, int cnt, int stop, int* wc, bool
     if (out == cnt) return cnt;
     cnt = out;
   }
-  // (not convex after that many passes: one thread's monotone chain, in place)
+  // (not convex after that many passes: one thread's monotone chain, in place. Sorted runs in
+  // random order come here, one permutation in 15 at 2048 points, 934 of them left at most of the
+  // 160 tried: the worst weighted row of 2048 took 169 us in all, where pairwise merges took 543)
   if (tid == 0) {
     int top = 0;
     for (int k = 0; k < cnt; ++k) {

@@ -392,7 +392,7 @@ struct ExpandArgs {
 struct LongPlan {
   int64_t tiles_per_row;  // expansion (and backward) tiles
   int64_t span0;          // elements per span (the first node level)
-  int rows_per_wave;      // > 1: rows of at most 2048 elements whose store is laid out in 64 / it spans each
+  int rows_per_wave;      // reported only. > 1: rows of at most 2048 elements, 64 / it spans in the store each
   int levels;
   int keep_level;  // the level whose vertex counts bound the final hulls' (see long_fit)
   int64_t batch;
