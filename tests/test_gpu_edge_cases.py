@@ -12,8 +12,7 @@ the sizes where they reach the merge levels, through the public API on the GPU:
 - blocks whose means all round to 1.0 in float32: the gradient takes its blocks from the hull,
   not from equal fitted values (reference tests/test_cuda.py:268-294, n = 500, 3000, 100 000);
 - rows of a batch are independent: rows of magnitude 1e30 beside ordinary ones, in every way
-  the kernels share a wave or a workgroup between rows (one row a lane, several rows a wave,
-  one row a wave), leave the ordinary rows' fits and gradients as they are alone.
+  the kernels lay rows out (one row a lane, a wave or a workgroup a row), leave the ordinary rows' fits and gradients as they are alone.
 """
 
 from __future__ import annotations
@@ -168,8 +167,7 @@ def test_gradient_blocks_from_the_hull(n: int) -> None:
 
 
 # (batch, n): rows of 32 one a lane (short kernel); 64 one a lane in batches of 8192 ("packed");
-# 128 in a batch of 2 (16 spans a row, 4 rows a wave), 300 in 64 (4 rows a wave), 2000 in 1000
-# (2 rows a wave); 5000 one row a wave
+# 128 and 300 a wave a row; 2000 and 5000 a workgroup of up to 256 and 512 threads a row
 INDEPENDENCE_SHAPES = [(1000, 32), (8192, 64), (2, 128), (64, 300), (1000, 2000), (4, 5000)]
 
 

@@ -243,19 +243,20 @@ def test_float32_chunk_joints_keep_the_fit_monotone(kind: str) -> None:
     assert float(np.abs(got - want).max()) <= tolerance(y) + rounding
 
 
-@pytest.mark.parametrize(("batch", "n"), [(1, 4_000_000), (300, 40_000), (600, 10_000), (3000, 1000), (9000, 100)])
+@pytest.mark.parametrize(("batch", "n"), [(1, 4_000_000), (80, 100_000), (300, 40_000), (1100, 20_000)])
 def test_float32_repair_chain_gives_the_same_hulls(batch: int, n: int) -> None:
     # The repair finishes a row with a sequential monotone chain after a cascade of removals
-    # longer than its pass limit; the REPAIR_CHAIN hint takes that form at once (through the
-    # check and repair launches for one row, in the last merge launch for 300, in the span
-    # kernel's waves or the first merge launch for 600 x 10000 (one row a wave), 3000 x 1000 (two
-    # rows a wave) and 9000 x 100 (eight)). Both keep the lower hull of the stored points, so fit
-    # and partition are the passes' bit for bit.
+    # longer than its pass limit; the REPAIR_CHAIN hint takes that form at once (through the check
+    # and repair launches for 1 and 80 rows, in the last merge launch's workgroups of 256 threads
+    # for 300 and of 64 for 1100; rows of one group, built on their stored values, have no repair
+    # but at the joints of merged chunks). Both keep the lower hull of the stored points, so fit and
+    # partition are the passes' bit for bit.
     say(f"float32 repair chain: {batch} weighted near-collinear rows of {n}")
     rng = np.random.default_rng(13)
     i = np.arange(n, dtype=np.float64)
     y = torch.from_numpy((1e3 + 1e-3 * i + 1e-7 * rng.standard_normal((batch, n))).astype(np.float32)).cuda()
     w = torch.from_numpy(np.exp(8 * rng.random((batch, n))).astype(np.float32)).cuda()
+    assert _ext.geometry(batch, n, True)["levels"] >= 2
     a, sa, bad_a, _ = _ext.fit(y, w, True, True, True)
     b, sb, bad_b, _ = _ext.fit(y, w, True, True, True, hints=_ext.REPAIR_CHAIN)
     assert bad_a is False and bad_b is False
@@ -266,8 +267,8 @@ def test_float32_repair_chain_gives_the_same_hulls(batch: int, n: int) -> None:
 
 # --- exact ties with inexact cross products ------------------------------------------------------
 
-# (batch, n): short rows, one row a lane ("packed"), several rows a wave, one row a wave, and rows
-# whose spans go through one, two and three merge launches
+# (batch, n): short rows, one row a lane ("packed"), one group a row in a wave and in a workgroup, and
+# rows whose groups go through one and two merge launches
 TIE_SHAPES = [(5, 6), (5, 30), (9000, 60), (300, 600), (3, 3000), (1, 100_002), (1, 3 * 2**20)]
 
 

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_util import check_fit, gpu_fit
+from gpu_util import check_fit, gpu_fit, tolerance
 from test_gpu_tiles import gpu_grads
 from torchisotonic_amd import _ext
 
@@ -72,13 +72,17 @@ def test_groups(n: int, weighted: bool, dtype: type) -> None:
 @pytest.mark.parametrize("n", [200, 3000, 20_000])
 def test_margin_over_every_height(n: int) -> None:
     # one value so large that the margin drops nothing by chords: every rise is a candidate, and
-    # the exact neighbour tests decide (compared as the fit: sums past the value round it away)
+    # the exact neighbour tests decide. Before the value, whose sums it is not in, fit and start
+    # bits are exact to those elements' own magnitude; from it on sums round the others away.
     rng = np.random.default_rng(n)
     for dtype in (np.float32, np.float64):
         y = np.stack([rows("mixed", n, rng) for _ in range(3)]).astype(dtype)
-        got, _ = gpu_fit(y)
-        want, _ = oracle.pava(y.astype(np.float64), acc="f64")
+        got, starts = gpu_fit(y)
+        want, want_starts = oracle.pava(y.astype(np.float64), acc="f64")
         assert float(np.abs(got - want).max()) <= 4 * np.finfo(dtype).eps * 1e25
+        before = slice(0, n // 3)
+        assert float(np.abs(got - want)[:, before].max()) <= tolerance(y[:, before])
+        np.testing.assert_array_equal(starts[:, : n // 3 + 1], want_starts[:, : n // 3 + 1])
 
 
 @pytest.mark.parametrize(("n", "batches"), [(1100, (4, 3000)), (2001, (4, 3000)), (2500, (4, 132, 600)),

@@ -1,4 +1,4 @@
-"""Rows longer than 32 elements (the span kernel, merges and tiled expansion) on the GPU against
+"""Rows longer than 32 elements (the group and span kernels, merges and tiled expansion) on the GPU against
 the oracle: the reference's lane/chunk edge shapes and adversarial patterns (reference
 tests/test_cuda.py:31-134, 224-265) restated for the HIP path."""
 
@@ -411,16 +411,15 @@ def test_many_rows_of_one_span(batch: int, n: int) -> None:
 
 @pytest.mark.parametrize(("batch", "n"), [(9_000, 100), (8_192, 256), (2_000, 512), (3_000, 1000), (5_000, 1500)])
 def test_several_rows_a_wave(batch: int, n: int) -> None:
-    # rows of at most 2048 elements: one small workgroup a row, or one row a lane of the span
-    # kernel
-    print(f"rows a wave batch={batch} n={n}", flush=True)
+    # rows of at most 2048 elements in batches of thousands: a wave or a small workgroup a row
+    print(f"short groups batch={batch} n={n}", flush=True)
     check_many_rows(batch, n)
 
 
-# (batch, n) of one merge level, one row a wave: the wave that builds a row's final hull also
-# writes its tile records, start bits and fit. Rows with a vertex at every element have more
-# edges than the wave's table of edge values holds (about 3.5k-4.8k), so it is restaged within
-# the row; n = 2049 is one element past the packed expansion's rows.
+# (batch, n) of one group a row: the workgroup that builds a row's hull also writes its tile
+# records, start bits and fit. Rows with a vertex at every element overflow its slots: the overflow
+# kernel's workgroup merges and expands them, from a table of edge values that is restaged within
+# the row; n = 2049 is one element past the groups that hold every point.
 ONE_LEVEL_SHAPES = [(600, 10_000), (700, 5_000), (2_100, 2_049)]
 
 
@@ -582,16 +581,21 @@ def chord_rows(rows: int, n: int, dtype: type, weighted: bool, seed: int) -> tup
 @pytest.mark.parametrize("increasing", [True, False])
 @pytest.mark.parametrize("weighted", [False, True])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_candidate_filter_same_bits(dtype: type, weighted: bool, increasing: bool) -> None:
-    # Small and large batches of rows of one group (600 and 3000 rows of 5000), whose points clearly
-    # above a chord drop before the exact tests. The same rows in
+@pytest.mark.parametrize(("n", "small", "big", "levels"), [(40, 9000, 140_000, 0), (5000, 600, 3000, 1)])
+def test_candidate_filter_same_bits(n: int, small: int, big: int, levels: int, dtype: type, weighted: bool,
+                                    increasing: bool) -> None:
+    # Rows of 40 elements, one a lane of the span kernel: a grid of at most two waves a SIMD (9000
+    # rows) runs its stronger candidate test, which drops points lying clearly above the chord of
+    # their neighbours two elements away; 140000 rows run without it. And rows of 5000, one group
+    # each, in two batches of one kernel. The same rows in
     # both give the same bits, and the oracle's fit (and, but for the rows over 24 decades, whose
     # sums round differently in any order, its partition).
     from torchisotonic_amd import _ext
 
-    n, small, big = 5000, 600, 3000
-    print(f"candidate filter dtype={np.dtype(dtype).name} weighted={weighted} increasing={increasing}", flush=True)
-    assert _ext.geometry(small, n, weighted) == _ext.geometry(big, n, weighted)
+    print(f"candidate filter n={n} dtype={np.dtype(dtype).name} weighted={weighted} increasing={increasing}", flush=True)
+    geo, geo_big = _ext.geometry(small, n, weighted), _ext.geometry(big, n, weighted)
+    assert geo["levels"] == geo_big["levels"] == levels
+    assert levels == 0 or geo == geo_big  # (rows one a lane: the span only lays out the store)
     y, w, kind = chord_rows(small, n, dtype, weighted, 11 + weighted + 2 * increasing)
     yb, wb, _ = chord_rows(big, n, dtype, weighted, 5)
     yb[:small] = y
