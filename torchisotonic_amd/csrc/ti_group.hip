@@ -25,13 +25,13 @@
 // holds (rising data, where most points are vertices) are built a chunk at a time and merged in
 // global memory by reference to the chunks' hulls (merge_global), by a second launch.
 //
-// What bounds it: VALU issue, about 1400 instructions a wave of 2048 weighted float32 elements (20
-// an element), and the latency of the load, three barriers and the candidates' rounds at two
-// workgroups a CU. One lane a span of 80 to 256 elements with a stack in LDS, the form before, was
-// bound by the chain of each stack operation. Forward calls, before and now: 20000 rows of 200
-// float32 107 -> 36 us; 10000 of 1000 131 -> 53 us; 1000 of 5000 60 -> 26 us, weighted float64 79
-// -> 68 us; 500 of 20000 120 -> 55 us; one weighted row of 1e8 (the kernel) 346 -> 240 us; rising
-// rows, all overflowing (1000 of 10000, a vertex at every element) 468 -> 178 us.
+// What bounds it: VALU issue, about 1500 instructions a wave of 2048 weighted float32 elements, and
+// the latency of the load, three barriers and the candidates' rounds at two workgroups a CU. One
+// lane a span of 80 to 256 elements with a stack in LDS, the form before, was bound by the chain of
+// each stack operation. Forward calls, before and now: 20000 rows of 200 float32 107 -> 36 us; 10000
+// of 1000 131 -> 56 us; 1000 of 5000 60 -> 27 us, weighted float64 81 -> 51 us; 500 of 20000 120 ->
+// 60 us; one weighted row of 1e8 (the kernel) 346 -> 233 us; rising rows, all overflowing (1000 of
+// 10000, a vertex at every element) 468 -> 187 us.
 #include <algorithm>
 
 #include "ti_common.h"
@@ -624,14 +624,14 @@ __global__ __launch_bounds__(NT, 4) void group_kernel(GroupArgs a) {
 // The groups of more candidates than slots (kOverflow): the points at every rise, a chunk of spans
 // at a time, each chunk's hull to its spans' slots in the group's frame, then those merged by
 // reference (merge_global). A workgroup a group, or several, which share its chunks, where groups
-// are few. Where none overflowed (noisy data) the launch is one read of the counts. (A kernel of its own: in group_kernel its registers would
-// halve every group's occupancy. Few threads a workgroup, as most of the merge keeps a few busy,
-// and up to eight workgroups a CU.)
+// are few. Where none overflowed (noisy data) the launch is one read of the counts. (A kernel of
+// its own: in group_kernel its registers would halve every group's occupancy. Few threads a
+// workgroup, as most of the merge keeps a few busy, and up to four workgroups a CU.)
 //
 // What bounds it: a chunk's rounds and the merge's chains of reads. With a workgroup a group
-// whatever their number, and float64 in 128 threads of 8 elements: one rising row of 16384 166 us
-// (weighted float64 377), now 128 (154); 200 of them 203 (484), now 209 (289); 1000 weighted
-// float64 ones of 5000 317, now 253.
+// whatever their number, and float64 in 128 threads of 8 elements: one weighted rising row of 16384
+// 166 us (float64 377), now 128 (154); 200 of them 203 (484), now 207 (289); 1000 float64 ones of
+// 5000 317, now 253 (float64: with the conversion of float32 inputs).
 template <typename T, bool W, int NT, int E, bool MAP>
 __global__ __launch_bounds__(NT, 4) void overflow_kernel(GroupArgs a) {
   constexpr bool PR = sizeof(T) == 8;
