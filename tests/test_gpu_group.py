@@ -109,6 +109,35 @@ def test_overflowing_groups_shared_by_workgroups(n: int, batches: tuple[int, ...
             np.testing.assert_array_equal(starts, np.tile(first[1], (b // 4, 1)))
 
 
+def test_overflowing_groups_replayed() -> None:
+    # the count of a group's workgroups starts from zero in every replay of a captured call, whether
+    # the group overflowed in the replay before or not
+    import torch
+
+    import torchisotonic_amd
+
+    print("overflowing groups in a graph", flush=True)
+    n = 9001
+    rng = np.random.default_rng(4)
+    data = [np.stack([rows(k, n, rng) for k in kinds]) for kinds in
+            (("rise", "drops", "rise"), ("noise", "rise", "noise"), ("rise", "rise", "drops"), ("noise", "noise", "noise"))]
+    data = [torch.from_numpy(d.astype(np.float32)).cuda() for d in data]
+    y = data[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torchisotonic_amd.isotonic(y)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        fit = torchisotonic_amd.isotonic(y)
+    for k in (0, 0, 1, 3, 2, 0):
+        y.copy_(data[k])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(fit, torchisotonic_amd.isotonic(data[k]))
+
+
 @pytest.mark.parametrize("n", [200, 512, 2048, 3840, 5000, 16384, 33_000])
 @pytest.mark.parametrize("weighted", [False, True])
 def test_sums_over_threads_carry_their_rounding(n: int, weighted: bool) -> None:

@@ -869,8 +869,10 @@ hipError_t group_launch(GroupArgs a, hipStream_t stream) {
   region = std::max(region, a.expand_at + (a.expand ? 64 + 2 * words4 * 4 + a.cap * tb : 0));
   region = (region + 63) & ~63;
   a.xp.lds_bytes = region;
+  const bool may_overflow = a.cap < a.g_elems + 3;
+  if (may_overflow && a.chunk * a.span0 % E != 0) return hipErrorInvalidConfiguration;  // (see overflow_shape)
   const hipError_t e = launch_lds(group_kernel<T, W, NT, E, MAP>, a, grid, a.nt, group_head_bytes(NW) + region, stream);
-  if (e != hipSuccess || a.cap >= a.g_elems + 3) return e;
+  if (e != hipSuccess || !may_overflow) return e;
   return overflow_launch<T, W, MAP>(a, stream);
 }
 
